@@ -63,6 +63,27 @@ static int check_weight(const PackedDesc &w)
     return EP_OK;
 }
 
+// Rows above which f32 group scales (a fine-tuned store's, which the small-M
+// kernels do not read) run on the prefill tiles rather than the generic
+// ones: 4-bit 2048 x 6144 at M = 5 / 32 / 48: 92.6 / 97.1 / 113.2 -> 24.0 /
+// 27.4 / 31.5 us, 6144 x 2048 at M = 16: 36.9 -> 18.3 us, 8-bit 4096^2 at
+// M = 8: 87.4 -> 24.1 us (the tiles split K over idle CUs and look up
+// conflict-free copies of the table).
+constexpr int64_t kTileRowsMin = 4;
+
+// The workspace without which a call cannot run: any M may land on the MFMA
+// path (shapes the GEMV does not serve), so the per-row exponent buffer is
+// always requested; 2..64 rows may take the split-K path and its partial
+// sums.
+size_t matmul_workspace_least(int64_t M, int64_t N, int64_t K, int levels)
+{
+    size_t need = mfma_workspace(M);
+    const size_t b = (M >= 2 && M <= 64) ? skinny_workspace(M, N, K, levels) : 0;
+    const size_t c = M > 64 ? prefill_workspace(M, N, K, levels) : 0;
+    need = need > b ? need : b;
+    return need > c ? need : c;
+}
+
 }  // namespace ep
 
 using namespace ep;
@@ -100,14 +121,9 @@ int ep_hip_available(void)
 size_t ep_dequant_matmul_workspace(int64_t M, int64_t N, int64_t K, int levels, int group)
 {
     (void)group;
-    // Any M may land on the MFMA path (shapes the GEMV does not serve), so
-    // the per-row exponent buffer is always requested; 2..64 rows may take
-    // the split-K path and its partial sums.
-    size_t need = mfma_workspace(M);
-    const size_t b = (M >= 2 && M <= 64) ? skinny_workspace(M, N, K, levels) : 0;
-    const size_t c = M > 64 ? prefill_workspace(M, N, K, levels) : 0;
-    need = need > b ? need : b;
-    return need > c ? need : c;
+    const size_t need = matmul_workspace_least(M, N, K, levels);
+    const size_t t = M > kTileRowsMin && M <= 64 ? prefill_workspace(M, N, K, levels) : 0;
+    return need > t ? need : t;
 }
 
 int ep_dequant_matmul(const void *x, int x_dtype, int64_t ldx, const uint8_t *packed,
@@ -141,6 +157,9 @@ int ep_dequant_matmul(const void *x, int x_dtype, int64_t ldx, const uint8_t *pa
     if (skinny_serves(w, xa, M))
         return launch_skinny(w, xa, M, ya, workspace, workspace_bytes, s);
     if (M > 64 && prefill_serves(w, xa, M))
+        return launch_prefill(w, xa, M, ya, workspace, workspace_bytes, s);
+    if (M > kTileRowsMin && M <= 64 && w.scale_dtype == EP_F32 && prefill_serves(w, xa, M) &&
+        workspace_bytes >= prefill_workspace(M, N, K, levels))
         return launch_prefill(w, xa, M, ya, workspace, workspace_bytes, s);
     if (mfma_serves(w, xa, M))
         return launch_mfma(w, xa, M, ya, workspace, workspace_bytes, s);

@@ -188,6 +188,10 @@ int blas_gemm_f32out(int ta, int tb, int64_t m, int64_t n, int64_t k, int ab_dty
                      int64_t lda, const void *B, int64_t ldb, float *D, int64_t ldd, float alpha,
                      void *ws, size_t ws_bytes, hipStream_t stream);
 
+// Bytes without which a dequant-matmul of this shape is refused (abi.cpp);
+// ep_dequant_matmul_workspace asks for what its fastest route uses.
+size_t matmul_workspace_least(int64_t M, int64_t N, int64_t K, int levels);
+
 // Checks a HIP call; on failure records the error and returns EP_ERR_HIP.
 #define EP_HIP_CHECK(expr)                                                                 \
     do {                                                                                   \

@@ -68,7 +68,7 @@ int ep_dequant_matmul_noalloc(const void *x, int x_dtype, int64_t ldx, const uin
     if (M < 0 || N < 0 || K < 0)
         return set_error(EP_ERR_ARG, "noalloc: negative shape M=%lld N=%lld K=%lld",
                          (long long)M, (long long)N, (long long)K);
-    const size_t need = ep_dequant_matmul_workspace(M, N, K, levels, group);
+    const size_t need = matmul_workspace_least(M, N, K, levels);
     if (need > kScratchBytes)
         return set_error(EP_ERR_WORKSPACE,
                          "noalloc: M=%lld N=%lld K=%lld needs %zu bytes of workspace, the static "

@@ -1,7 +1,8 @@
-// Prefill (M > 64 rows) fused codebook dequant-matmul on gfx950 MFMA.
+// Prefill (M > 64 rows; f32 group scales: M > 4) fused codebook dequant-matmul on gfx950 MFMA.
 //
 // y[M, N] = x[M, K] . W[N, K]^T, W[n, k] = cb[idx[n, k]] * scale[n, k / group],
-// for row counts where the contraction is compute-bound.  Reference
+// for row counts where the contraction is compute-bound (and, with f32 group
+// scales, from a few rows up).  Reference
 // behaviour: the table kernel epure/kernels/_triton.py:54-107 (fp16 operands,
 // fp32 accumulation) and, for the dense tile, materialize(float16)
 // (runtime.py:78-89): the weight enters the product as fp16(fp16(cb) * fp16(scale)).
@@ -28,6 +29,10 @@
 //    replicated 32 times (lane & 31 reads its own copy: no bank conflicts),
 //    addressed by one v_perm of the packed word, then the group scale is
 //    applied in fp16 (v_pk_mul_f16);
+//  * group scales are read as stored, fp16 or f32 (SF32: a fine-tuned
+//    store's, rounded to fp16 where they enter the product as the generic
+//    tiles did): 4-bit 2048 x 6144 at M = 201 with f32 scales 139.7 -> 41.5
+//    us against mm_kernel, 6144 x 2048 at M = 2048 131.8 -> 99.9 us;
 //  * activations are converted once to fp16 after the exact per-row
 //    power-of-two rescale by a pre-kernel (pf_prep_kernel, into the
 //    workspace) and staged in LDS as they are, double buffered: step k + 1
@@ -162,9 +167,10 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-template <int BITS, int BM, int PD, int NT, int WAVES, bool GR = false>
+template <int BITS, int BM, int PD, int NT, int WAVES, bool GR, bool SF32>
 __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
 {
+    constexpr int SB = SF32 ? 4 : 2;             // bytes of a group scale
     constexpr int MT = BM / 32;                  // 32-row M tiles per wave
     constexpr int THREADS = WAVES * 64;
     constexpr int TPR = THREADS / BM;            // staging threads per activation row
@@ -206,7 +212,7 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
         gstart = tl[1];
         gcount = tl[2];
         a.packed += (int64_t)e * a.estride_w;
-        a.scale = (const char *)a.scale + e * a.estride_s * 2;
+        a.scale = (const char *)a.scale + e * a.estride_s * SB;
     }
     const auto rx = buffer_rsrc(a.x, a.xbytes), rw = buffer_rsrc(a.packed, a.wbytes);
     const auto rs = buffer_rsrc(a.scale, a.sbytes), rcb = buffer_rsrc(a.cb, a.cbbytes);
@@ -237,7 +243,7 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
             wlo[nt][l] = n < a.N ? (uint32_t)n * a.row_bytes + (uint32_t)(BITS == 4 ? kl / 2 : kl) : kPfOut;
             // the group divides 64 or is 64 * 2^i: the piece's group is the
             // step's (kt * gk_mul) >> gk_shift plus kl / group
-            slo[nt][l] = n < a.N ? (uint32_t)(((int64_t)n * a.lds + kl / a.group) * 2) : kPfOut;
+            slo[nt][l] = n < a.N ? (uint32_t)(((int64_t)n * a.lds + kl / a.group) * SB) : kPfOut;
         }
     }
     auto kstep_ok = [&](int kt) { return kt < nk && kt < kt0 + a.ksteps; };
@@ -250,13 +256,16 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
     auto issue_w = [&](int kt, u32x4_t (&w)[NT][WL], uint32_t (&sr)[NT][WL]) {
         const bool kok = kstep_ok(kt);
         const uint32_t kw = kok ? (uint32_t)(kt * (BITS == 4 ? kPfBK / 2 : kPfBK)) : kPfOut;
-        const uint32_t kg = kok ? (uint32_t)(((kt * a.gk_mul) >> a.gk_shift) * 2) : kPfOut;
+        const uint32_t kg = kok ? (uint32_t)(((kt * a.gk_mul) >> a.gk_shift) * SB) : kPfOut;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int l = 0; l < WL; ++l) {
                 w[nt][l] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(wlo[nt][l] + kw), 0, 0);
-                sr[nt][l] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(slo[nt][l] + kg), 0, 0);
+                if constexpr (SF32)
+                    sr[nt][l] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(slo[nt][l] + kg), 0, 0);
+                else
+                    sr[nt][l] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(slo[nt][l] + kg), 0, 0);
             }
     };
 
@@ -350,7 +359,7 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
         for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
             for (int l = 0; l < WL; ++l) {
-                const f16_t s16 = f16_from_bits((uint16_t)sc[nt][l]);
+                const f16_t s16 = SF32 ? (f16_t)__uint_as_float(sc[nt][l]) : f16_from_bits((uint16_t)sc[nt][l]);
                 const f16x2_t s2 = (f16x2_t){s16, s16};
 #pragma unroll
                 for (int wd = 0; wd < 4; ++wd) {
@@ -453,7 +462,7 @@ PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
     PfPlan p;
     if (bits == 4) {
         // measured: 128 x 2 tiles lead from M = 1024, 128 x 1 at 256..1023
-        p.bm = M >= EP_PF_BIG4_M ? 128 : 64;
+        p.bm = M >= EP_PF_BIG4_M ? 128 : M > 32 ? 64 : 32;
         p.nt = M >= EP_PF_BIG4_M && M < 1024 ? 1 : 2;
         p.pd = p.bm == 128 && p.nt == 2 ? 2 : 4;
         p.waves = M >= EP_PF_BIG4_M ? 8 : 4;
@@ -463,7 +472,7 @@ PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
         p.nt = 1;
         p.waves = 8;
     } else {
-        p.bm = 64;
+        p.bm = M > 32 ? 64 : 32;
         p.pd = 3;
         p.nt = 2;
         p.waves = 4;
@@ -488,21 +497,27 @@ PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
 }
 
 template <int BITS, int BM, int PD, int NT, int WAVES>
-int pf_launch(const PfArgs &a, const PfPlan &p, hipStream_t s)
+int pf_launch(const PfArgs &a, const PfPlan &p, bool sf32, hipStream_t s)
 {
     constexpr int BN = WAVES * 32 * NT;
     const dim3 grid((unsigned)((a.N + BN - 1) / BN), (unsigned)((a.M + BM - 1) / BM), (unsigned)p.S);
-    hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES>), grid, dim3(WAVES * 64), 0, s, a);
+    if (sf32)
+        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, false, true>), grid, dim3(WAVES * 64), 0, s, a);
+    else
+        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, false, false>), grid, dim3(WAVES * 64), 0, s, a);
     EP_HIP_CHECK(hipGetLastError());
     return EP_OK;
 }
 
 template <int BITS, int BM, int PD, int NT, int WAVES>
-int pf_launch_grouped(const PfArgs &a, unsigned tiles_y, hipStream_t s)
+int pf_launch_grouped(const PfArgs &a, unsigned tiles_y, bool sf32, hipStream_t s)
 {
     constexpr int BN = WAVES * 32 * NT;
     const dim3 grid((unsigned)((a.N + BN - 1) / BN), tiles_y, 1u);
-    hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, true>), grid, dim3(WAVES * 64), 0, s, a);
+    if (sf32)
+        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, true, true>), grid, dim3(WAVES * 64), 0, s, a);
+    else
+        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, true, false>), grid, dim3(WAVES * 64), 0, s, a);
     EP_HIP_CHECK(hipGetLastError());
     return EP_OK;
 }
@@ -528,6 +543,7 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
                            void *ws, hipStream_t stream)
 {
     const int bits = w.bits();
+    const bool sf32 = w.scale_dtype == EP_F32;
     int *rexp = (int *)ws;
     f16_t *xh = (f16_t *)((char *)ws + (T * 4 + 255) / 256 * 256);
     hipLaunchKernelGGL(pf_prep_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, stream, x.ptr, x.dtype,
@@ -536,7 +552,7 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     PfArgs a{};
     a.xbytes = (uint32_t)(T * w.K * 2);
     a.wbytes = (uint32_t)(w.N * (bits == 4 ? w.K / 2 : w.K));
-    a.sbytes = (uint32_t)(((w.N - 1) * w.ld_scale + (w.K + w.group - 1) / w.group) * 2);
+    a.sbytes = (uint32_t)(((w.N - 1) * w.ld_scale + (w.K + w.group - 1) / w.group) * (sf32 ? 4 : 2));
     a.cbbytes = (uint32_t)(w.levels * (w.cb_dtype == EP_F32 ? 4 : 2));
     a.x = xh;
     a.ldx = w.K;
@@ -575,21 +591,21 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     if (bits == 4) {
         if (bm == 128) {
             a.ksteps = ks(4);
-            return pf_launch_grouped<4, 128, 4, 1, 8>(a, tiles_y, stream);
+            return pf_launch_grouped<4, 128, 4, 1, 8>(a, tiles_y, sf32, stream);
         }
         a.ksteps = ks(4);
         if (bm == 32)
-            return pf_launch_grouped<4, 32, 4, 2, 4>(a, tiles_y, stream);
-        return pf_launch_grouped<4, 64, 4, 2, 4>(a, tiles_y, stream);
+            return pf_launch_grouped<4, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
+        return pf_launch_grouped<4, 64, 4, 2, 4>(a, tiles_y, sf32, stream);
     }
     if (bm == 128) {
         a.ksteps = ks(EP_PF_PD8);
-        return pf_launch_grouped<8, 128, EP_PF_PD8, 1, 8>(a, tiles_y, stream);
+        return pf_launch_grouped<8, 128, EP_PF_PD8, 1, 8>(a, tiles_y, sf32, stream);
     }
     a.ksteps = ks(3);
     if (bm == 32)
-        return pf_launch_grouped<8, 32, 3, 2, 4>(a, tiles_y, stream);
-    return pf_launch_grouped<8, 64, 3, 2, 4>(a, tiles_y, stream);
+        return pf_launch_grouped<8, 32, 3, 2, 4>(a, tiles_y, sf32, stream);
+    return pf_launch_grouped<8, 64, 3, 2, 4>(a, tiles_y, sf32, stream);
 }
 
 bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
@@ -597,7 +613,7 @@ bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
     const int bits = w.bits();
     if (M < 1 || M > ((int64_t)1 << 24) || w.N < 1 || w.K < kPfBK || w.K % kPfBK != 0)
         return false;
-    if (w.scale_dtype != EP_F16 || w.group % (bits == 4 ? 32 : 16) != 0)
+    if ((w.scale_dtype != EP_F16 && w.scale_dtype != EP_F32) || w.group % (bits == 4 ? 32 : 16) != 0)
         return false;
     // groups that divide the 64-wide k step or are 64 * 2^i (others: the
     // generic MFMA path)
@@ -606,7 +622,7 @@ bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
     const int esz = x.dtype == EP_F32 ? 4 : 2;
     const int64_t rb = bits == 4 ? w.K / 2 : w.K;
     const int64_t G = (w.K + w.group - 1) / w.group;
-    if (w.N * rb > kPfOut || ((M - 1) * x.ld + w.K) * esz > kPfOut || ((w.N - 1) * w.ld_scale + G) * 2 > kPfOut)
+    if (w.N * rb > kPfOut || ((M - 1) * x.ld + w.K) * esz > kPfOut || ((w.N - 1) * w.ld_scale + G) * (w.scale_dtype == EP_F32 ? 4 : 2) > kPfOut)
         return false;
     if (((uintptr_t)w.packed & 15) != 0 || ((uintptr_t)x.ptr & 15) != 0)
         return false;
@@ -628,6 +644,7 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
     if (!prefill_serves(w, x, M))
         return EP_DECLINE_SHAPE;
     const int bits = w.bits();
+    const bool sf32 = w.scale_dtype == EP_F32;
     const PfPlan p = pf_plan(bits, M, w.N, w.K);
     const bool partials = p.S > 1;
     const size_t ex = (size_t)((M * 4 + 255) / 256 * 256);
@@ -643,7 +660,7 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
     PfArgs a{};
     a.xbytes = (uint32_t)(M * w.K * 2);
     a.wbytes = (uint32_t)(w.N * (bits == 4 ? w.K / 2 : w.K));
-    a.sbytes = (uint32_t)(((w.N - 1) * w.ld_scale + (w.K + w.group - 1) / w.group) * 2);
+    a.sbytes = (uint32_t)(((w.N - 1) * w.ld_scale + (w.K + w.group - 1) / w.group) * (sf32 ? 4 : 2));
     a.cbbytes = (uint32_t)(w.levels * (w.cb_dtype == EP_F32 ? 4 : 2));
     a.x = xh;
     a.ldx = w.K;
@@ -671,12 +688,14 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
     a.part = partials ? (float *)((char *)ws + ex + xhb) : nullptr;
     int rc;
     if (bits == 4)
-        rc = p.nt == 1 ? pf_launch<4, 128, 4, 1, 8>(a, p, stream)
-             : p.bm == 128 ? pf_launch<4, 128, 2, 2, 8>(a, p, stream)
-                           : pf_launch<4, 64, 4, 2, 4>(a, p, stream);
+        rc = p.nt == 1 ? pf_launch<4, 128, 4, 1, 8>(a, p, sf32, stream)
+             : p.bm == 128 ? pf_launch<4, 128, 2, 2, 8>(a, p, sf32, stream)
+             : p.bm == 64  ? pf_launch<4, 64, 4, 2, 4>(a, p, sf32, stream)
+                           : pf_launch<4, 32, 4, 2, 4>(a, p, sf32, stream);
     else
-        rc = p.nt == 1 ? pf_launch<8, 128, EP_PF_PD8, 1, 8>(a, p, stream)
-                       : pf_launch<8, 64, 3, 2, 4>(a, p, stream);
+        rc = p.nt == 1   ? pf_launch<8, 128, EP_PF_PD8, 1, 8>(a, p, sf32, stream)
+             : p.bm == 64 ? pf_launch<8, 64, 3, 2, 4>(a, p, sf32, stream)
+                          : pf_launch<8, 32, 3, 2, 4>(a, p, sf32, stream);
     if (rc != EP_OK || !partials)
         return rc;
     return launch_split_reduce(a.part, p.S, M, w.N, y, stream);

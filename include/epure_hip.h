@@ -74,8 +74,8 @@ int ep_hip_available(void);
 const char *ep_last_error(void);
 
 /*
- * Workspace bytes ep_dequant_matmul needs for this shape (a few bytes per
- * activation row).  The caller passes at least this much.
+ * Workspace bytes ep_dequant_matmul needs for this shape.  The caller passes
+ * at least this much.
  */
 size_t ep_dequant_matmul_workspace(int64_t M, int64_t N, int64_t K, int levels, int group);
 
@@ -99,7 +99,8 @@ size_t ep_dequant_matmul_workspace(int64_t M, int64_t N, int64_t K, int levels, 
  * split-K over slices of 2048 or 4096 values with each wave's activations
  * held in registers;
  * split-K over slices of at most 1024 otherwise; the splits' f32 partials
- * summed in split order), dequant-to-LDS + MFMA above.  Each reads the
+ * summed in split order), MFMA tiles with the weights dequantized in
+ * registers above (with f32 group scales from M = 5).  Each reads the
  * packed bytes exactly once per launch.
  */
 int ep_dequant_matmul(const void *x, int x_dtype, int64_t ldx,

@@ -191,3 +191,22 @@ def test_batch1_8bit_long_k_stays_on_the_gemv():
     torch.cuda.synchronize()
     us = e0.elapsed_time(e1) / 20 * 1e3
     assert us < 60.0, f"{us:.1f} us per launch"
+
+
+@pytest.mark.parametrize("levels,group", [(16, 128), (16, 32), (256, 128), (256, 16)])
+@pytest.mark.parametrize("m,n,k", [(5, 515, 1024), (32, 300, 512), (33, 257, 4096), (64, 256, 64),
+                                   (65, 130, 2048), (161, 513, 1088), (1024, 300, 512)])
+def test_f32_scales_on_the_tiles(levels, group, m, n, k):
+    """f32 group scales (a fine-tuned store's) on the tile kernel at the edges
+    of its row tiles (32, 64, 128), with K split and whole, against the f64
+    product of its operands: fp16(fp16(cb) * fp16(scale)) and x, exact in
+    fp16.  What is left is the f32 sum of K <= 4096 products in some order,
+    at most K * 2^-24 = 2.5e-4 of the sum of their magnitudes and far less of
+    the result: held to 1e-4 of it."""
+    _, packed, scale, cb, _ = make(n, k, levels, group, seed=m + n + k)
+    f32 = (np.asarray(scale, np.float32) * np.float32(1.0003)).astype(np.float32)
+    s = PackedWeight((n, k), packed, f32, cb.astype(np.float32), group, levels).to(DEV)
+    assert s.scale.dtype == torch.float32
+    _, x = x_bf16(m, k, m)
+    want = (x.double() @ s.materialize(torch.float16).double().t()).cpu().numpy()
+    assert_close(run(s, x).cpu().numpy(), want, 1e-4)
