@@ -5,6 +5,8 @@ mapped (both carry the soname ``libamdhip64.so.7``): streams and device
 pointers from torch are then valid handles for the library.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -106,11 +108,25 @@ _SIGS = {
 XSRC_PLAIN, XSRC_RMSNORM, XSRC_SWIGLU = 0, 1, 2
 
 lib = None
+call = None  # the native call path (csrc/torch_call.cpp), bound to ``lib``
 LOAD_ERROR = None
+TORCH_PATH = os.path.join(os.path.dirname(LIB_PATH), "epure_torch.so")
+
+
+def _load_call(handle):
+    """The extension that calls ``handle``'s matmul entry points on tensors."""
+    loader = importlib.machinery.ExtensionFileLoader("epure_torch", TORCH_PATH)
+    ext = importlib.util.module_from_spec(
+        importlib.util.spec_from_file_location("epure_torch", TORCH_PATH, loader=loader))
+    addr = lambda name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value  # noqa: E731
+    ext.bind(addr("ep_dequant_matmul_workspace"), addr("ep_dequant_matmul"),
+             addr("ep_dequant_matmul_bwd_workspace"), addr("ep_dequant_matmul_bwd"),
+             addr("ep_last_error"), getattr(torch._C, "_cuda_getCurrentRawStream", None))
+    return ext
 
 
 def _load():
-    global lib, LOAD_ERROR
+    global lib, call, LOAD_ERROR
     if lib is not None or LOAD_ERROR is not None:
         return lib
     try:
@@ -121,6 +137,7 @@ def _load():
             fn.argtypes = args
         if handle.ep_abi_version() != ABI_VERSION:
             raise ImportError(f"{LIB_NAME} ABI {handle.ep_abi_version()} != {ABI_VERSION}")
+        call = _load_call(handle)
         lib = handle
     except Exception as exc:                    # noqa: BLE001 - recorded and re-raised by callers
         LOAD_ERROR = exc

@@ -106,49 +106,15 @@ def _hot(store):
 
 def forward(x2, h, out=None, accumulate=False):
     """Launch y = x2 @ W^T for a 2-D ``x2``.  Returns y, or None on decline."""
-    M, K = x2.shape
-    xdt = _abi.dtype_code(x2.dtype)
-    if out is None:
-        out = torch.empty((M, h.N), device=x2.device, dtype=x2.dtype)
-    ydt = _abi.dtype_code(out.dtype)
-    ws_bytes = _abi.lib.ep_dequant_matmul_workspace(M, h.N, K, h.levels, h.group)
-    ws = torch.empty(ws_bytes, device=x2.device, dtype=torch.uint8) if ws_bytes else None
-    rc = _abi.lib.ep_dequant_matmul(
-        x2.data_ptr(), xdt, x2.stride(0),
-        h.packed.data_ptr(), h.scale.data_ptr(), h.scale_dt, h.ld_scale,
-        h.cb.data_ptr(), h.cb_dt, h.levels, h.group,
-        M, h.N, K,
-        out.data_ptr(), ydt, out.stride(0), _abi.FLAG_ACCUMULATE if accumulate else 0,
-        ws.data_ptr() if ws is not None else None, ws_bytes, _abi.stream_handle(x2.device))
-    return out if _abi.check(rc, "ep_dequant_matmul") else None
+    return _abi.call.matmul(x2, h.packed, h.scale, h.cb, h.N, h.levels, h.group, out, accumulate)
 
 
 def backward(gy2, x2, h, need_x=True, need_cb=True, need_scale=True, gx_dtype=None):
     """Fused backward; returns (grad_x, grad_cb, grad_scale) or None on decline.
 
     grad_x has ``gx_dtype`` (default: x's dtype)."""
-    M, N = gy2.shape
-    K = x2.shape[1]
-    gx = torch.empty((M, K), device=x2.device, dtype=gx_dtype or x2.dtype) if need_x else None
-    G = (K + h.group - 1) // h.group
-    gcb = torch.empty(h.levels, device=x2.device, dtype=torch.float32) if need_cb else None
-    gsc = torch.empty((N, G), device=x2.device, dtype=torch.float32) if need_scale else None
-    ws_bytes = _abi.lib.ep_dequant_matmul_bwd_workspace(M, N, K, h.levels, h.group)
-    ws = torch.empty(ws_bytes, device=x2.device, dtype=torch.uint8) if ws_bytes else None
-    rc = _abi.lib.ep_dequant_matmul_bwd(
-        gy2.data_ptr(), _abi.dtype_code(gy2.dtype), gy2.stride(0),
-        x2.data_ptr(), _abi.dtype_code(x2.dtype), x2.stride(0),
-        h.packed.data_ptr(), h.scale.data_ptr(), h.scale_dt, h.ld_scale,
-        h.cb.data_ptr(), h.cb_dt, h.levels, h.group,
-        M, N, K,
-        gx.data_ptr() if gx is not None else None,
-        _abi.dtype_code(gx.dtype if gx is not None else x2.dtype), K,
-        gcb.data_ptr() if gcb is not None else None,
-        gsc.data_ptr() if gsc is not None else None, G,
-        ws.data_ptr() if ws is not None else None, ws_bytes, _abi.stream_handle(x2.device))
-    if not _abi.check(rc, "ep_dequant_matmul_bwd"):
-        return None
-    return gx, gcb, gsc
+    return _abi.call.backward(gy2, x2, h.packed, h.scale, h.cb, h.N, h.levels, h.group, need_x,
+                              need_cb, need_scale, _abi.dtype_code(gx_dtype or x2.dtype))
 
 
 class _PackedLinearFn(torch.autograd.Function):
@@ -183,7 +149,21 @@ class _PackedLinearFn(torch.autograd.Function):
 
 def linear(x, store):
     """``x @ dequant(store).T`` on the GPU, or ``None`` if unsupported."""
-    if not available() or not x.is_cuda or len(store.shape) != 2:
+    if not available() or len(store.shape) != 2:
+        return None
+    # an inference call on plain tensors: all of it in one native call, which
+    # reads pointers, strides and flags from the tensors of this call
+    own = store.__dict__
+    bufs = own.get("_buffers")
+    if bufs is not None:
+        pars = own["_parameters"]
+        packed, scale, cb = (bufs[a] if a in bufs else pars.get(a)
+                             for a in ("packed", "scale", "cb"))
+        y = _abi.call.linear(x, packed, scale, cb, own["out_features"], own["in_features"],
+                             own["levels"], own["group"], SERVE_F32)
+        if y is not NotImplemented:
+            return y
+    if not x.is_cuda:
         return None
     if x.dtype not in (torch.float16, torch.bfloat16) and not (
             SERVE_F32 and x.dtype == torch.float32):

@@ -225,7 +225,8 @@ class PackedLinear(nn.Module):
         if len(s.shape) != 2 or s.__dict__.get("_force_materialize", False):
             return None
         if x.is_cuda:
-            rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
+            k = x.shape[-1]
+            rows = x.numel() // k if k else 0
             return cuda_kernel.linear(x, s) if rows < _DENSE_ABOVE else None
         if s.levels > 16:
             return None
