@@ -160,6 +160,18 @@ EP_DEV float xor32_sum(float v)
     const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
+// Sums of lanes l and l ^ 32 of two values: a's in lanes 0..31, b's in 32..63.
+EP_DEV float half_sums32(float a, float b)
+{
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// Sums of lanes l and l ^ 16: a's in the even 16-lane groups, b's in the odd.
+EP_DEV float half_sums16(float a, float b)
+{
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
 EP_DEV float xor16_max(float v)
 {
     const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);

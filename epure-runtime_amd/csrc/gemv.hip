@@ -622,9 +622,17 @@ __global__ void __launch_bounds__(512) gemv_lut_kernel(GemvArgs a)
 // waited (config 0: 5.30 -> 4.59 us per launch; weights issued between the
 // staging and the table build: 4.85).  SC32: f32 group scales; otherwise one
 // 16-bit load per scale (fp16 or bf16), not the two halves of a word
-// (4.61 -> 4.48 us).
-template <int BITS, int XDT, int S, bool SC32, int MT>
-__global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES) gemv_row_kernel(GemvArgs a)
+// (4.61 -> 4.48 us).  LOOP: layers of several rounds of workgroups build the
+// table and stage the activations once per resident workgroup and stream a
+// contiguous share of the row blocks, the next block's loads in flight
+// during this one's products: the per-block prologue (64 KiB of table for 32
+// KiB of weights) was most of a long layer's time, and then the rows' lane
+// sums (now shared by a wave's rows: 12 instead of 48 operations for four).
+// 4-bit 151936 x 2048 50.5 -> 33.3 us (4.8 TB/s; 42.2 before the shared
+// sums), 32768 x 8192 57.2 -> 28.9, 8192^2 16.1 -> 10.5, 8-bit 28672 x 4096
+// 33.0 -> 24.6.
+template <int BITS, int XDT, int S, bool SC32, int MT, bool LOOP>
+__global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES, LOOP ? 4 : 1) gemv_row_kernel(GemvArgs a)
 {
     constexpr int NW = EP_GEMV_ROW_WAVES;       // waves per workgroup
     constexpr int NT = 64 * NW;
@@ -668,7 +676,10 @@ __global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES) gemv_row_kernel(GemvAr
         xbase += (int64_t)blockIdx.y * a.ldx * ESZ;
         yp = (char *)yp + (int64_t)blockIdx.y * a.ldy * (a.y_dtype == EP_F32 ? 4 : 2);
     }
-    const int row0 = (int)blockIdx.x * ROWS + wave * RW;
+    // LOOP: this workgroup's contiguous share of the row blocks; else the one
+    const int nblk = (N + ROWS - 1) / ROWS;
+    const int blk0 = LOOP ? (int)((int64_t)nblk * blockIdx.x / gridDim.x) : (int)blockIdx.x;
+    const int blk1 = LOOP ? (int)((int64_t)nblk * (blockIdx.x + 1) / gridDim.x) : blk0 + 1;
 
     // ---- the activation chunk and codebook loads (the weights follow the
     // table build); chunk ch is chunk ch % NCH of activation row ch / NCH
@@ -757,10 +768,12 @@ __global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES) gemv_row_kernel(GemvAr
     }
     __builtin_amdgcn_sched_barrier(0);
     // weights: load i covers row r = i / LPR, slabs 4 (i % LPR) .. + 3
-    u32x4_t wq[NL];
-    uint32_t sraw[NL];  // the scale's bits: f32 (SC32) or fp16 / bf16
-    {
+    constexpr int SETS = LOOP ? 2 : 1;
+    u32x4_t wq[SETS][NL];
+    uint32_t sraw[SETS][NL];  // the scale's bits: f32 (SC32) or fp16 / bf16
+    auto issue = [&](int blk, u32x4_t (&wq)[NL], uint32_t (&sraw)[NL]) {
         const auto *sp = (const __attribute__((address_space(1))) uint16_t *)scale;
+        const int row0 = blk * ROWS + wave * RW;
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int row = row0 + i / LPR;
@@ -779,7 +792,8 @@ __global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES) gemv_row_kernel(GemvAr
             else
                 sraw[i] = sp[e];
         }
-    }
+    };
+    issue(blk0, wq[0], sraw[0]);
     __builtin_amdgcn_sched_barrier(0);  // the weight loads go out before the barrier
     lds_barrier();
 
@@ -817,6 +831,8 @@ __global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES) gemv_row_kernel(GemvAr
 
     // ---- dot products: load i adds to row i / LPR of every activation row
     const uint32_t lane4 = ((uint32_t)lane & 31) << 2;  // the lane's table copy
+    auto block = [&](int blk, const u32x4_t (&wq)[NL], const uint32_t (&sraw)[NL]) {
+    const int row0 = blk * ROWS + wave * RW;
     float acc[RW][MT];
 #pragma unroll
     for (int r = 0; r < RW; ++r)
@@ -871,21 +887,52 @@ __global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES) gemv_row_kernel(GemvAr
         for (int m = 0; m < MT; ++m)
             acc[r][m] = fmaf(HL ? part[m] + plo[m] : part[m], scr * fexp[xj][m], acc[r][m]);
     }
-    // ---- each row's sums inside the wave; lane 0 stores them
+    // ---- each row's sum inside the wave: the rows share the two halving
+    // steps (the halves of two rows meet in one swap and one add), so four
+    // rows cost little more than one; 16-lane group q ends with row rq
+    const int q = lane >> 4;
+    const int rq = RW == 4 ? ((q & 1) << 1) | (q >> 1) : RW == 2 ? q >> 1 : 0;
+    const bool lead = (lane & (RW == 4 ? 15 : RW == 2 ? 31 : 63)) == 0;
 #pragma unroll
-    for (int r = 0; r < RW; ++r)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const float v = wave_sum(acc[r][m]);
-            const int row = row0 + r;
-            if (lane == 0 && row < N && m < a.M) {
-                const int64_t off = (int64_t)m * a.ldy + row;
-                float o = v;
-                if (a.accumulate)
-                    o += load_as_f32(yp, a.y_dtype, off);
-                store_from_f32(yp, a.y_dtype, off, o);
-            }
+    for (int m = 0; m < MT; ++m) {
+        float v;
+        if constexpr (RW == 4)
+            v = half_sums16(half_sums32(acc[0][m], acc[1][m]), half_sums32(acc[2][m], acc[3][m]));
+        else if constexpr (RW == 2)
+            v = xor16_sum(half_sums32(acc[0][m], acc[1][m]));
+        else
+            v = xor16_sum(xor32_sum(acc[0][m]));
+        v += dpp_mov<0x128>(v);
+        v += dpp_mov<0x124>(v);
+        v += dpp_mov<0x4e>(v);
+        v += dpp_mov<0xb1>(v);
+        const int row = row0 + rq;
+        if (lead && row < N && m < a.M) {
+            const int64_t off = (int64_t)m * a.ldy + row;
+            if (a.accumulate)
+                v += load_as_f32(yp, a.y_dtype, off);
+            store_from_f32(yp, a.y_dtype, off, v);
         }
+    }
+    };
+    if constexpr (!LOOP) {
+        block(blk0, wq[0], sraw[0]);
+    } else {
+        // the next block's loads go out before this block's products; past
+        // the share they repeat its last block's (cached, never used)
+        for (int blk = blk0;; blk += 2) {
+            issue(blk + 1 < blk1 ? blk + 1 : blk, wq[1], sraw[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            block(blk, wq[0], sraw[0]);
+            if (blk + 1 >= blk1)
+                break;
+            issue(blk + 2 < blk1 ? blk + 2 : blk + 1, wq[0], sraw[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            block(blk + 1, wq[1], sraw[1]);
+            if (blk + 2 >= blk1)
+                break;
+        }
+    }
 }
 
 // Any shape, any stride, any M: one wave per output row, fp32 arithmetic
@@ -1182,13 +1229,36 @@ static bool row_serves(const GemvArgs &a, int bits, int xdt, int64_t M)
     return row_serves_shape(bits, a.row_bytes, xdt, M);
 }
 
+// Workgroups of the row GEMV that a CU's 160 KiB of LDS holds (at most two
+// are wanted): the pair table and the staged activation row.
+constexpr int row_wgs_per_cu(int bits, int S)
+{
+    const int lds = kTabDwords * 4 + S * 16 * ((bits == 4 ? 16 : 8) * 4 + 4) + 16;
+    return 160 * 1024 / lds >= 2 ? 2 : 1;
+}
+
 template <int BITS, int XDT, int S, int MT>
 static void launch_row_sc(const GemvArgs &a, dim3 g, dim3 b, hipStream_t stream)
 {
+    if constexpr (MT == 1 && XDT != EP_F32) {
+        // the loop from 1.75 rounds of resident workgroups (4-bit 14336 x
+        // 4096: 11.4 -> 10.2 us; at one round 16384 x 2048 ran 7.2 -> 8.2),
+        // rows above 16 slabs, whose own loads are deeper, from three (8-bit
+        // 8192 x 7168 at two rounds: 16.5 -> 17.0)
+        const unsigned wgs = (unsigned)(row_wgs_per_cu(BITS, S) * device_cus());
+        if (!a.gidx && 4 * g.x >= (S <= 16 ? 7 : 12) * wgs) {
+            const dim3 gl(wgs);
+            if (a.scale_dtype == EP_F32)
+                hipLaunchKernelGGL((gemv_row_kernel<BITS, XDT, S, true, MT, true>), gl, b, 0, stream, a);
+            else
+                hipLaunchKernelGGL((gemv_row_kernel<BITS, XDT, S, false, MT, true>), gl, b, 0, stream, a);
+            return;
+        }
+    }
     if (a.scale_dtype == EP_F32)
-        hipLaunchKernelGGL((gemv_row_kernel<BITS, XDT, S, true, MT>), g, b, 0, stream, a);
+        hipLaunchKernelGGL((gemv_row_kernel<BITS, XDT, S, true, MT, false>), g, b, 0, stream, a);
     else
-        hipLaunchKernelGGL((gemv_row_kernel<BITS, XDT, S, false, MT>), g, b, 0, stream, a);
+        hipLaunchKernelGGL((gemv_row_kernel<BITS, XDT, S, false, MT, false>), g, b, 0, stream, a);
 }
 
 template <int BITS, int XDT, int S>

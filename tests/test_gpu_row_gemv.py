@@ -124,3 +124,44 @@ def test_row_gemv_several_rows_strided_accumulate(out_dtype):
     """Activation rows further apart than K, results added into y."""
     case_m(4, 1000, 4096, 16, torch.bfloat16, seed=91, out_dtype=out_dtype, accumulate=True, ld_pad=96)
     case_m(2, 1000, 4096, 256, torch.bfloat16, seed=92, out_dtype=out_dtype, accumulate=True, ld_pad=96)
+
+
+@pytest.mark.parametrize("levels,k,n", [
+    (16, 2048, 28671), (16, 2048, 28673), (16, 4096, 14353), (16, 8192, 3585), (16, 8192, 8191),
+    (16, 16384, 6145), (256, 1024, 28705), (256, 2048, 14337), (256, 4096, 7171), (256, 7168, 12289)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_row_gemv_streams_row_blocks(levels, k, n, xdt):
+    """Layers of several rounds of workgroups, each streaming a share of the
+    row blocks: counts of blocks that no share divides, shares of odd and
+    even length, and a last block cut by N, against the f64 product of the
+    operands (fp16 codebook values, f32 scales and sums: x is exact in both
+    types)."""
+    s = PackedWeight((n, k), *_random_store(n, k, levels), 128, levels).to(DEV)
+    x = _random_x(k, xdt)
+    y = cuda.forward(x, cuda._hot(s), out=torch.empty((1, n), device=DEV, dtype=torch.float32))
+    assert y is not None, f"declined: {_abi.last_error()}"
+    idx = s.packed.view(n, -1)
+    if levels == 16:
+        idx = torch.stack((idx & 15, idx >> 4), dim=-1).view(n, k)
+    w = s.cb.double()[idx.long()] * s.scale.double().repeat_interleave(128, dim=1)
+    want = (x.double() @ w.t())
+    err = (y.double() - want).abs().max() / want.pow(2).mean().sqrt()
+    # f32 sums of K products and an exact per-32 rescale of fp16-sized x:
+    # K * 2^-24 = 1e-3 of the summed magnitudes at the longest row bounds it;
+    # the sums' rounding is random and stays far below
+    assert err < 1e-4, f"{float(err):.2e}"
+
+
+def _random_store(n, k, levels):
+    g = torch.Generator()
+    g.manual_seed(n + k)
+    packed = torch.randint(0, 256, (n * k // (2 if levels == 16 else 1),), generator=g, dtype=torch.uint8)
+    cb = torch.sort(torch.randn(levels, generator=g)).values.half().float()
+    scale = (torch.randn(n, k // 128, generator=g).abs() * 0.02 + 1e-3).half()
+    return packed, scale, cb
+
+
+def _random_x(k, xdt):
+    g = torch.Generator()
+    g.manual_seed(k)
+    return torch.randn(1, k, generator=g).to(DEV).to(xdt)
