@@ -32,13 +32,24 @@
 //  * group scales are read as stored, fp16 or f32 (SF32: a fine-tuned
 //    store's, rounded to fp16 where they enter the product as the generic
 //    tiles did): 4-bit 2048 x 6144 at M = 201 with f32 scales 139.7 -> 41.5
-//    us against mm_kernel, 6144 x 2048 at M = 2048 131.8 -> 99.9 us;
+//    us against mm_kernel, 6144 x 2048 at M = 2048 131.8 -> 99.9 us (36.2 and
+//    88.4 since);
 //  * activations are converted once to fp16 after the exact per-row
 //    power-of-two rescale by a pre-kernel (pf_prep_kernel, into the
 //    workspace) and staged in LDS as they are, double buffered: step k + 1
 //    is stored while step k is multiplied;
 //  * weight loads run PD steps ahead in registers (buffer loads: a row past
 //    N or a step past K reads zeros without touching memory);
+//  * the step is software pipelined and its LDS reads are spread between its
+//    MFMAs (step, interleave): in one phase after another the matrix cores
+//    and the LDS were each under half busy (28% / 48% at 8-bit 2048 x 14336
+//    x 4096).  Next to bind were the L1's line accesses (65% busy): staging
+//    loads of eight threads per row read whole lines, and with groups of a
+//    multiple of 128 one scale load serves two steps (a load of 32 rows'
+//    scales touches 32 lines).  Together 8-bit 2048 x 14336 x 4096: 390 ->
+//    354 us, 2048 x 4096 x 14336: 366 -> 319, 512 x 14336 x 4096: 106 -> 97;
+//    4-bit 2048 x 14336 x 4096: 309 -> 281, 333 x 6656 x 2560: 44.7 -> 40.7
+//    (graph replays, all launches);
 //  * when the grid of (N / (32 WAVES NT)) x (M / BM) workgroups cannot fill the device,
 //    K is split and the f32 partials are summed in split order by the
 //    reduction shared with the small-M path (deterministic).
@@ -73,7 +84,7 @@ struct PfArgs {
     int K;
     int group;
     int gk_mul, gk_shift;  // k step kt starts in group (kt * gk_mul) >> gk_shift
-    int ksteps;   // k steps per split (a multiple of the unroll)
+    int ksteps;   // k steps per split (even)
     const int *rexp;
     uint32_t xbytes, wbytes, sbytes, cbbytes;
     void *y;
@@ -167,19 +178,19 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-template <int BITS, int BM, int PD, int NT, int WAVES, bool GR, bool SF32>
+template <int BITS, int BM, int PD, int NT, int WAVES, bool GR, bool SF32, bool G128>
 __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
 {
     constexpr int SB = SF32 ? 4 : 2;             // bytes of a group scale
     constexpr int MT = BM / 32;                  // 32-row M tiles per wave
     constexpr int THREADS = WAVES * 64;
-    constexpr int TPR = THREADS / BM;            // staging threads per activation row
-    constexpr int VPT = kPfBK / TPR;             // values per staging thread and step
     constexpr int XE = 2;  // activations: fp16, pre-scaled per row (pf_prep_kernel)
-    constexpr int XP = VPT * XE / 16;            // 16-byte pieces per staging thread
+    constexpr int XROWS = THREADS / 8;           // activation rows per staging load (8 threads a row)
+    constexpr int XP = BM / XROWS;               // 16-byte pieces per staging thread and step
     constexpr int WL = BITS == 4 ? 1 : 2;        // 16-byte weight loads per lane, N tile and step
-    constexpr int NB = (PD > 2 ? PD : 2) + 1;    // register sets (weights PD, activations 2 steps ahead)
-    static_assert(VPT % 8 == 0, "staging in 8-value pieces");
+    constexpr int NB = PD;                       // register sets of weights
+    constexpr int UN = 4;  // unrolled steps (a multiple of PD; two register sets of activations and of scale pairs)
+    static_assert(UN % PD == 0 && BM % XROWS == 0, "register sets rotate with the unroll");
     static_assert(THREADS >= 256, "one table entry per thread");
     static_assert(BM <= 128, "two activation buffers in the table's gaps");
 
@@ -219,20 +230,28 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
 
     // ---- first loads: codebook, row exponents, step 0's activations
     const uint32_t cbraw = __builtin_amdgcn_raw_buffer_load_b32(rcb, tid * 4, 0, 0);
-    const int xr = tid / TPR, xq = tid % TPR;
-    int xm;
-    if constexpr (GR)
-        xm = xr < gcount ? a.perm[gstart + xr] : -1;
-    else
-        xm = m0 + xr < a.M ? m0 + xr : -1;
-    const int ex = *(const __attribute__((address_space(1))) int *)(a.rexp + (xm >= 0 ? xm : 0));
+    // row r of the tile: its token (row of x), -1 past M or the expert's run
+    auto row_token = [&](int r) -> int {
+        if constexpr (GR)
+            return r < gcount ? a.perm[gstart + r] : -1;
+        else
+            return m0 + r < a.M ? m0 + r : -1;
+    };
+    const int xr = tid / 8, xq = tid % 8;  // staging: piece xq of rows xr, xr + XROWS, ..
+    const int em = tid < BM ? row_token(tid) : -1;
+    const int ex = *(const __attribute__((address_space(1))) int *)(a.rexp + (em >= 0 ? em : 0));
 
     // Load offsets = a per-lane part fixed for the whole loop (kPfOut for a
     // row past M or N) + a per-step part that is uniform (kPfOut for a step
     // past K or the split): one add per load.  Both parts stay below 2^31,
     // so a sum with either at kPfOut is past the buffer and reads zeros
     // (the bounds check covers the per-lane offset, which holds the sum).
-    const uint32_t xlo = xm >= 0 ? (uint32_t)(((int64_t)xm * a.ldx + xq * VPT) * XE) : kPfOut;
+    uint32_t xlo[XP];
+#pragma unroll
+    for (int p = 0; p < XP; ++p) {
+        const int xm = row_token(xr + p * XROWS);
+        xlo[p] = xm >= 0 ? (uint32_t)(((int64_t)xm * a.ldx + xq * 8) * XE) : kPfOut;
+    }
     uint32_t wlo[NT][WL], slo[NT][WL];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -246,36 +265,55 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
             slo[nt][l] = n < a.N ? (uint32_t)(((int64_t)n * a.lds + kl / a.group) * SB) : kPfOut;
         }
     }
-    auto kstep_ok = [&](int kt) { return kt < nk && kt < kt0 + a.ksteps; };
+    const int kend = kt0 + a.ksteps < nk ? kt0 + a.ksteps : nk;
     auto issue_x = [&](int kt, u32x4_t (&xv)[XP]) {
-        const uint32_t ks = kstep_ok(kt) ? (uint32_t)(kt * kPfBK * XE) : kPfOut;
+        const uint32_t ks = kt < kend ? (uint32_t)(kt * kPfBK * XE) : kPfOut;
 #pragma unroll
         for (int p = 0; p < XP; ++p)
-            xv[p] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(xlo + ks + 16 * p), 0, 0);
+            xv[p] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(xlo[p] + ks), 0, 0);
+    };
+    auto load_scale = [&](uint32_t off) -> uint32_t {
+        if constexpr (SF32)
+            return __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0);
+        else
+            return __builtin_amdgcn_raw_buffer_load_b16(rs, (int)off, 0, 0);
+    };
+    auto group_off = [&](int kt) -> uint32_t {
+        return kt < kend ? (uint32_t)(((kt * a.gk_mul) >> a.gk_shift) * SB) : kPfOut;
     };
     auto issue_w = [&](int kt, u32x4_t (&w)[NT][WL], uint32_t (&sr)[NT][WL]) {
-        const bool kok = kstep_ok(kt);
-        const uint32_t kw = kok ? (uint32_t)(kt * (BITS == 4 ? kPfBK / 2 : kPfBK)) : kPfOut;
-        const uint32_t kg = kok ? (uint32_t)(((kt * a.gk_mul) >> a.gk_shift) * SB) : kPfOut;
+        const uint32_t kw = kt < kend ? (uint32_t)(kt * (BITS == 4 ? kPfBK / 2 : kPfBK)) : kPfOut;
+        const uint32_t kg = group_off(kt);
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int l = 0; l < WL; ++l) {
                 w[nt][l] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(wlo[nt][l] + kw), 0, 0);
-                if constexpr (SF32)
-                    sr[nt][l] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(slo[nt][l] + kg), 0, 0);
-                else
-                    sr[nt][l] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(slo[nt][l] + kg), 0, 0);
+                if constexpr (!G128)
+                    sr[nt][l] = load_scale(slo[nt][l] + kg);
             }
     };
+    // G128 (groups of a multiple of 128): one scale serves the two steps
+    // kt, kt + 1 (kt - kt0 even) and both pieces of each
+    auto issue_s = [&](int kt, uint32_t (&sr)[NT]) {
+        const uint32_t kg = group_off(kt);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            sr[nt] = load_scale(slo[nt][0] + kg);
+    };
 
-    // NB register sets, rotated with static indices: weights run PD steps
+    // register sets, rotated with static indices: weights up to PD steps
     // ahead, activations two steps ahead (stored to LDS one step ahead)
-    u32x4_t xv[NB][XP];
+    u32x4_t xv[2][XP];
     u32x4_t wb[NB][NT][WL];
     uint32_t sb[NB][NT][WL];
+    uint32_t sp[2][NT];  // G128: the scales of two pairs of steps
     issue_x(kt0, xv[0]);
     issue_x(kt0 + 1, xv[1]);
+    if constexpr (G128) {
+        issue_s(kt0, sp[0]);
+        issue_s(kt0 + 2, sp[1]);
+    }
 #pragma unroll
     for (int d = 0; d < PD; ++d)
         issue_w(kt0 + d, wb[d], sb[d]);
@@ -288,14 +326,17 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
     auto store_x = [&](const u32x4_t (&v4)[XP], int q) {
 #pragma unroll
         for (int p = 0; p < XP; ++p)
-            *(u32x4_t *)((char *)tab + xs_off(q, xr, xq * XP + p)) = v4[p];
+            *(u32x4_t *)((char *)tab + xs_off(q, xr + p * XROWS, xq)) = v4[p];
     };
 
     // codebook -> fp16 -> the replicated table; step 0's activations -> LDS
     if (tid < 256)
         s_cbraw[tid] = cbraw;
-    if (tid < BM)
-        s_e[tid] = 0;
+    if (tid < BM) {
+        s_e[tid] = em >= 0 ? ex : 0;
+        if constexpr (GR)
+            s_row[tid] = em;
+    }
     lds_barrier();
     {
         float c = 0.0f;
@@ -321,12 +362,6 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
                 row[i] = (u32x4_t){v, v, v, v};
         }
     }
-    if (tid % TPR == 0) {
-        if (xm >= 0)
-            s_e[xr] = ex;
-        if constexpr (GR)
-            s_row[xr] = xm;
-    }
     store_x(xv[0], 0);
     lds_barrier();
 
@@ -340,78 +375,127 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
                 acc[mt][nt][r] = 0.0f;
 
     const uint32_t c4 = (uint32_t)(lane & 31) << 2;  // the lane's table copy
-    // One step (register set r = (kt - kt0) % NB): issue step kt + 2's
-    // activations and step kt + PD's weights, multiply step kt, store step
-    // kt + 1's activations.
-    auto step = [&](int kt, auto rc) {
-        constexpr int r = decltype(rc)::value;
-        issue_x(kt + 2, xv[(r + 2) % NB]);
-        issue_w(kt + PD, wb[(r + PD) % NB], sb[(r + PD) % NB]);
-        // the loads above stay here, ahead of the work below (the scheduler
-        // would otherwise sink them next to their use)
-        __builtin_amdgcn_sched_barrier(0);
-        // activation buffer of step kt: static when the unroll is even
-        const int q = NB % 2 == 0 ? (r & 1) : ((kt - kt0) & 1);
-        u32x4_t (&wc)[NT][WL] = wb[r];
-        uint32_t (&sc)[NT][WL] = sb[r];
-        f16x2_t pr[NT][16];
+    // Operand s of step register set r: the 8 weights of each lane for MFMA
+    // sub-step s, in two parts with the MFMAs of another sub-step between
+    // them: the table lookups, and their pairs times the group scale.
+    constexpr int LQ = BITS == 4 ? 4 : 8;  // lookups per sub-step and N tile
+    f16x2_t pr[NT][16];
+    uint32_t tq[NT][LQ];
+    auto lookup = [&](const u32x4_t (&w)[NT][WL], int s) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int b = 0; b < LQ; ++b) {
+                const uint32_t word = BITS == 4 ? w[nt][0][s] : w[nt][WL == 2 ? s / 2 : 0][2 * (s % 2) + b / 4];
+                tq[nt][b] = lds_read_u32(tab, __builtin_amdgcn_perm(word, c4, kSelByte[b % 4]));
+            }
+    };
+    auto scaled = [&](int r, int s) {  // operand s of unrolled step r
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
+            const uint32_t raw = G128 ? sp[(r / 2) % 2][nt] : sb[r % NB][nt][WL == 2 ? s / 2 : 0];
+            const f16_t s16 = SF32 ? (f16_t)__uint_as_float(raw) : f16_from_bits((uint16_t)raw);
+            const f16x2_t s2 = (f16x2_t){s16, s16};
 #pragma unroll
-            for (int l = 0; l < WL; ++l) {
-                const f16_t s16 = SF32 ? (f16_t)__uint_as_float(sc[nt][l]) : f16_from_bits((uint16_t)sc[nt][l]);
-                const f16x2_t s2 = (f16x2_t){s16, s16};
-#pragma unroll
-                for (int wd = 0; wd < 4; ++wd) {
-                    const uint32_t word = wc[nt][l][wd];
-                    if constexpr (BITS == 4) {
-#pragma unroll
-                        for (int b = 0; b < 4; ++b)
-                            pr[nt][wd * 4 + b] =
-                                as_f16x2(lds_read_u32(tab, __builtin_amdgcn_perm(word, c4, kSelByte[b]))) * s2;
-                    } else {
-                        const uint32_t t0 = lds_read_u32(tab, __builtin_amdgcn_perm(word, c4, kSelByte[0]));
-                        const uint32_t t1 = lds_read_u32(tab, __builtin_amdgcn_perm(word, c4, kSelByte[1]));
-                        const uint32_t t2 = lds_read_u32(tab, __builtin_amdgcn_perm(word, c4, kSelByte[2]));
-                        const uint32_t t3 = lds_read_u32(tab, __builtin_amdgcn_perm(word, c4, kSelByte[3]));
-                        pr[nt][l * 8 + wd * 2] = as_f16x2(__builtin_amdgcn_perm(t1, t0, 0x05040100u)) * s2;
-                        pr[nt][l * 8 + wd * 2 + 1] = as_f16x2(__builtin_amdgcn_perm(t3, t2, 0x05040100u)) * s2;
-                    }
-                }
-            }
+            for (int p = 0; p < 4; ++p)
+                pr[nt][4 * s + p] = as_f16x2(BITS == 4 ? tq[nt][p]
+                                                       : __builtin_amdgcn_perm(tq[nt][(2 * p + 1) % LQ], tq[nt][(2 * p) % LQ],
+                                                                               0x05040100u)) * s2;
         }
+    };
+    f16x8_t av[2][MT];
+    auto read_a = [&](int q, int s, f16x8_t (&v)[MT]) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            f16x8_t av[MT];
+        for (int mt = 0; mt < MT; ++mt)
+            v[mt] = *(const f16x8_t *)((const char *)tab + xs_off(q, mt * 32 + j, 4 * h + s));
+    };
+    auto mfmas = [&](int s, const f16x8_t (&v)[MT]) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const f16x8_t bv = {pr[nt][4 * s][0],     pr[nt][4 * s][1],     pr[nt][4 * s + 1][0],
+                                pr[nt][4 * s + 1][1], pr[nt][4 * s + 2][0], pr[nt][4 * s + 2][1],
+                                pr[nt][4 * s + 3][0], pr[nt][4 * s + 3][1]};
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                av[mt] = *(const f16x8_t *)((const char *)tab + xs_off(q, mt * 32 + j, 4 * h + s));
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[mt], bv, acc[mt][nt], 0, 0, 0);
+        }
+    };
+    // One step (r = (kt - kt0) % UN), software pipelined.  Beside the MFMAs
+    // of sub-step s run the activation reads of sub-step s + 1, the lookups
+    // of operand s - 1 of step kt + 1 (s = 0: operand 3 of step kt) and the
+    // scaling of the operand looked up a sub-step before; the step's one
+    // barrier sits before its last MFMAs.  The LDS reads are spread between
+    // the MFMAs (interleave): issued ahead of them, the eight waves' reads
+    // filled the LDS queue while the matrix cores waited, then the other way
+    // round (both under half busy).
+    auto interleave = [&]() {
+        constexpr int NM = MT * NT, ND = (MT + NT * LQ + NM - 1) / NM;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const f16x8_t bv = {pr[nt][4 * s][0],     pr[nt][4 * s][1],     pr[nt][4 * s + 1][0],
-                                    pr[nt][4 * s + 1][1], pr[nt][4 * s + 2][0], pr[nt][4 * s + 2][1],
-                                    pr[nt][4 * s + 3][0], pr[nt][4 * s + 3][1]};
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[mt], bv, acc[mt][nt], 0, 0, 0);
-            }
+        for (int i = 0; i < NM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                              // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, ND, 0);  // LDS reads
+            __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);                              // VALU
         }
         __builtin_amdgcn_sched_barrier(0);
-        store_x(xv[(r + 1) % NB], q ^ 1);
-        // LDS-only barrier: __syncthreads() would also wait for the loads
-        // in flight
+    };
+    auto step = [&](int kt, auto rc) {
+        constexpr int r = decltype(rc)::value;
+        constexpr int wc = r % NB, wn = (r + 1) % NB, q = r & 1;
+        issue_x(kt + 2, xv[q]);
+        __builtin_amdgcn_sched_barrier(0);
+        scaled(r, 2);
+        mfmas(0, av[0]);
+        read_a(q, 1, av[1]);
+        lookup(wb[wc], 3);
+        interleave();
+        scaled(r, 3);
+        mfmas(1, av[1]);
+        read_a(q, 2, av[0]);
+        lookup(wb[wn], 0);
+        interleave();
+        issue_w(kt + PD, wb[wc], sb[wc]);  // the set that operand 3 was the last of
+        if constexpr (G128 && r % 2 == 1)
+            issue_s(kt + 3, sp[r / 2]);  // two pairs on, into the pair this step ends
+        store_x(xv[q ^ 1], q ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        scaled(r + 1, 0);
+        mfmas(2, av[0]);
+        read_a(q, 3, av[1]);
+        lookup(wb[wn], 1);
+        interleave();
+        // LDS-only barrier: __syncthreads() would also wait for the loads in
+        // flight.  Every wave has read its operands of buffer q and stored
+        // its part of buffer q ^ 1.
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        scaled(r + 1, 1);
+        mfmas(3, av[1]);
+        read_a(q ^ 1, 0, av[0]);
+        lookup(wb[wn], 2);
+        interleave();
     };
 
-    // ksteps is a multiple of NB; steps past K read zeros and add nothing
-    for (int kt = kt0; kt < kt0 + a.ksteps; kt += NB) {
+    // operands 0 and 1 of the first step, the lookups of operand 2
+    lookup(wb[0], 0);
+    scaled(0, 0);
+    lookup(wb[0], 1);
+    scaled(0, 1);
+    lookup(wb[0], 2);
+    read_a(0, 0, av[0]);
+    // steps past the split's end load zeros and are not run
+    for (int kt = kt0;; kt += UN) {
         step(kt, std::integral_constant<int, 0>{});
+        if (kt + 1 >= kend)
+            break;
         step(kt + 1, std::integral_constant<int, 1>{});
+        if (kt + 2 >= kend)
+            break;
         step(kt + 2, std::integral_constant<int, 2>{});
-        if constexpr (NB > 3)
-            step(kt + 3, std::integral_constant<int, 3 % NB>{});
-        if constexpr (NB > 4)
-            step(kt + 4, std::integral_constant<int, 4 % NB>{});
+        if (kt + 3 >= kend)
+            break;
+        step(kt + 3, std::integral_constant<int, 3>{});
+        if (kt + 4 >= kend)
+            break;
     }
 
     // D[row][col] of a 32x32 tile: lane col + 32 * ((row / 4) % 2), register
@@ -441,7 +525,6 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
 }
 
 // Tile rows, weight prefetch depth and K split for a shape.
-// 8-bit tiling knobs (measured: weight prefetch depth 2-4 within 1%)
 // M from which the 8-wave 128-row tilings run (measured: 8-bit gains from
 // M = 128, 4-bit only above it)
 #ifndef EP_PF_BIG4_M
@@ -451,10 +534,10 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
 #define EP_PF_BIG8_M 128
 #endif
 #ifndef EP_PF_PD8
-#define EP_PF_PD8 3
+#define EP_PF_PD8 4
 #endif
 struct PfPlan {
-    int bm, pd, nt, waves, S, ksteps;
+    int bm, nt, waves, S, ksteps;
 };
 
 PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
@@ -464,20 +547,16 @@ PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
         // measured: 128 x 2 tiles lead from M = 1024, 128 x 1 at 256..1023
         p.bm = M >= EP_PF_BIG4_M ? 128 : M > 32 ? 64 : 32;
         p.nt = M >= EP_PF_BIG4_M && M < 1024 ? 1 : 2;
-        p.pd = p.bm == 128 && p.nt == 2 ? 2 : 4;
         p.waves = M >= EP_PF_BIG4_M ? 8 : 4;
     } else if (M >= EP_PF_BIG8_M) {
         p.bm = 128;
-        p.pd = EP_PF_PD8;
         p.nt = 1;
         p.waves = 8;
     } else {
         p.bm = M > 32 ? 64 : 32;
-        p.pd = 3;
         p.nt = 2;
         p.waves = 4;
     }
-    const int nb = (p.pd > 2 ? p.pd : 2) + 1;
     const int bn = p.waves * 32 * p.nt;
     const int64_t tiles = ((N + bn - 1) / bn) * ((M + p.bm - 1) / p.bm);
     const int nk = (int)(K / kPfBK);
@@ -489,8 +568,7 @@ PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
     int S = 1;
     while (tiles * S * 2 <= target && S < 8 && nk / (S * 2) >= 8)
         S *= 2;
-    int ks = (nk + S - 1) / S;
-    ks = (ks + nb - 1) / nb * nb;
+    const int ks = ((nk + S - 1) / S + 1) / 2 * 2;
     p.S = (nk + ks - 1) / ks;
     p.ksteps = ks;
     return p;
@@ -501,10 +579,12 @@ int pf_launch(const PfArgs &a, const PfPlan &p, bool sf32, hipStream_t s)
 {
     constexpr int BN = WAVES * 32 * NT;
     const dim3 grid((unsigned)((a.N + BN - 1) / BN), (unsigned)((a.M + BM - 1) / BM), (unsigned)p.S);
-    if (sf32)
-        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, false, true>), grid, dim3(WAVES * 64), 0, s, a);
-    else
-        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, false, false>), grid, dim3(WAVES * 64), 0, s, a);
+    const bool g128 = a.group % 128 == 0;
+    const auto kern = sf32 ? (g128 ? pf_kernel<BITS, BM, PD, NT, WAVES, false, true, true>
+                                   : pf_kernel<BITS, BM, PD, NT, WAVES, false, true, false>)
+                           : (g128 ? pf_kernel<BITS, BM, PD, NT, WAVES, false, false, true>
+                                   : pf_kernel<BITS, BM, PD, NT, WAVES, false, false, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(WAVES * 64), 0, s, a);
     EP_HIP_CHECK(hipGetLastError());
     return EP_OK;
 }
@@ -514,10 +594,12 @@ int pf_launch_grouped(const PfArgs &a, unsigned tiles_y, bool sf32, hipStream_t 
 {
     constexpr int BN = WAVES * 32 * NT;
     const dim3 grid((unsigned)((a.N + BN - 1) / BN), tiles_y, 1u);
-    if (sf32)
-        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, true, true>), grid, dim3(WAVES * 64), 0, s, a);
-    else
-        hipLaunchKernelGGL((pf_kernel<BITS, BM, PD, NT, WAVES, true, false>), grid, dim3(WAVES * 64), 0, s, a);
+    const bool g128 = a.group % 128 == 0;
+    const auto kern = sf32 ? (g128 ? pf_kernel<BITS, BM, PD, NT, WAVES, true, true, true>
+                                   : pf_kernel<BITS, BM, PD, NT, WAVES, true, true, false>)
+                           : (g128 ? pf_kernel<BITS, BM, PD, NT, WAVES, true, false, true>
+                                   : pf_kernel<BITS, BM, PD, NT, WAVES, true, false, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(WAVES * 64), 0, s, a);
     EP_HIP_CHECK(hipGetLastError());
     return EP_OK;
 }
@@ -583,29 +665,21 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     a.ntiles = ntiles;
     a.estride_w = w.N * (int64_t)a.row_bytes;
     a.estride_s = w.N * w.ld_scale;
-    // the whole K per workgroup: steps rounded up to the register-set count
-    auto ks = [&](int pd) {
-        const int nb = (pd > 2 ? pd : 2) + 1;
-        return (nk + nb - 1) / nb * nb;
-    };
+    a.ksteps = (nk + 1) / 2 * 2;  // the whole K per workgroup
     if (bits == 4) {
         if (bm == 128) {
-            a.ksteps = ks(4);
             return pf_launch_grouped<4, 128, 4, 1, 8>(a, tiles_y, sf32, stream);
         }
-        a.ksteps = ks(4);
         if (bm == 32)
             return pf_launch_grouped<4, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
         return pf_launch_grouped<4, 64, 4, 2, 4>(a, tiles_y, sf32, stream);
     }
     if (bm == 128) {
-        a.ksteps = ks(EP_PF_PD8);
         return pf_launch_grouped<8, 128, EP_PF_PD8, 1, 8>(a, tiles_y, sf32, stream);
     }
-    a.ksteps = ks(3);
     if (bm == 32)
-        return pf_launch_grouped<8, 32, 3, 2, 4>(a, tiles_y, sf32, stream);
-    return pf_launch_grouped<8, 64, 3, 2, 4>(a, tiles_y, sf32, stream);
+        return pf_launch_grouped<8, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
+    return pf_launch_grouped<8, 64, 4, 2, 4>(a, tiles_y, sf32, stream);
 }
 
 bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
@@ -694,8 +768,8 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
                            : pf_launch<4, 32, 4, 2, 4>(a, p, sf32, stream);
     else
         rc = p.nt == 1   ? pf_launch<8, 128, EP_PF_PD8, 1, 8>(a, p, sf32, stream)
-             : p.bm == 64 ? pf_launch<8, 64, 3, 2, 4>(a, p, sf32, stream)
-                          : pf_launch<8, 32, 3, 2, 4>(a, p, sf32, stream);
+             : p.bm == 64 ? pf_launch<8, 64, 4, 2, 4>(a, p, sf32, stream)
+                          : pf_launch<8, 32, 4, 2, 4>(a, p, sf32, stream);
     if (rc != EP_OK || !partials)
         return rc;
     return launch_split_reduce(a.part, p.S, M, w.N, y, stream);
