@@ -63,7 +63,7 @@ struct BwdArgs {
     float *gscale;
     int64_t ldgs;
     const int *rexp;     // [M] per-row exponents of gy
-    const f16_t *gy16;   // [M][N] fp16(gy * 2^-rexp), written by gy_prep_kernel
+    const f16_t *gy16;   // [M][N] fp16(gy * 2^-rexp), written by row_prep_kernel
     float *gc_part;      // [num dw workgroups][16]
     int dx_steps;        // contraction steps per dx split
     float *dx_part;      // [splits][M][K] f32 partials (null: one split, results go to gx)
@@ -92,58 +92,6 @@ EP_DEV void tr8x8(const u32x4_t (&r)[8], u32x4_t (&c)[8])
         for (int d = 0; d < 4; ++d)
             c[j][d] = __builtin_amdgcn_perm(r[2 * d + 1][j >> 1], r[2 * d][j >> 1],
                                             (j & 1) ? 0x07060302u : 0x05040100u);
-}
-
-// Per-row exponent of the largest |gy| (row_exponent) and the rescaled
-// fp16 copy of the row, converted once here instead of once per k tile of
-// the dx kernel: one wave per row of bf16 values, 16-byte loads, four in
-// flight per lane (rows are 16-byte aligned and N % 16 == 0); the second
-// pass re-reads the row from the caches.
-__global__ void __launch_bounds__(256)
-    gy_prep_kernel(const uint16_t *gy, int64_t ld, int M, int N, int *rexp, f16_t *gy16)
-{
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= M)
-        return;
-    const u32x4_t *p = (const u32x4_t *)(gy + (int64_t)row * ld);
-    const int pieces = N / 8;
-    float amax = 0.0f;
-    for (int i0 = lane; i0 < pieces; i0 += 256) {
-        u32x4_t v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            v[u] = i0 + 64 * u < pieces ? p[i0 + 64 * u] : (u32x4_t){0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                amax = fmaxf(amax, fmaxf(fabsf(__uint_as_float(v[u][t] << 16)),
-                                         fabsf(__uint_as_float(v[u][t] & 0xffff0000u))));
-    }
-    amax = wave_max(amax);
-    const int e = row_exponent(amax);
-    if (lane == 0)
-        rexp[row] = e;
-    const float pw = ldexpf(1.0f, -e);
-    f16x8_t *q = (f16x8_t *)(gy16 + (int64_t)row * N);
-    for (int i0 = lane; i0 < pieces; i0 += 256) {
-        u32x4_t v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            v[u] = i0 + 64 * u < pieces ? p[i0 + 64 * u] : (u32x4_t){0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            f16x8_t h;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                h[2 * t] = (f16_t)(__uint_as_float(v[u][t] << 16) * pw);
-                h[2 * t + 1] = (f16_t)(__uint_as_float(v[u][t] & 0xffff0000u) * pw);
-            }
-            if (i0 + 64 * u < pieces)
-                q[i0 + 64 * u] = h;
-        }
-    }
 }
 
 // grad_x[m, k] = sum_n gy[m, n] W[n, k] over a 128 x 128 (m, k) tile,
@@ -970,10 +918,10 @@ int launch_backward(const PackedDesc &w, const ActDesc &gy, const ActDesc &x, in
                 }
             }
             if (gx.ptr) {
-                hipLaunchKernelGGL(gy_prep_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, stream,
-                                   (const uint16_t *)gy.ptr, gy.ld, (int)M, (int)w.N, rexp, gy16);
-                EP_HIP_CHECK(hipGetLastError());
-                int rc = launch_dequant_tile(w, w16, EP_F16, w.K, stream);  // materialize(float16)
+                int rc = launch_row_prep(gy, M, w.N, rexp, gy16, stream);
+                if (rc != EP_OK)
+                    return rc;
+                rc = launch_dequant_tile(w, w16, EP_F16, w.K, stream);  // materialize(float16)
                 if (rc != EP_OK)
                     return rc;
                 // column-major: D (K x M) = W16 (K x N) . gy16 (N x M)
@@ -1022,9 +970,8 @@ int launch_backward(const PackedDesc &w, const ActDesc &gy, const ActDesc &x, in
         const size_t nwg_bytes = (size_t)((w.K + T - 1) / T) * ((w.N + T - 1) / T) * 16 * sizeof(float);
         f16_t *gy16 = (f16_t *)((char *)a.gc_part + nwg_bytes);
         a.gy16 = gy16;
-        hipLaunchKernelGGL(gy_prep_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, stream,
-                           (const uint16_t *)gy.ptr, gy.ld, (int)M, (int)w.N, (int *)ws, gy16);
-        EP_HIP_CHECK(hipGetLastError());
+        if (const int rc = launch_row_prep(gy, M, w.N, (int *)ws, gy16, stream); rc != EP_OK)
+            return rc;
         const int S = dx_splits(M, w.N, w.K);
         const int nsteps = (int)((w.N + CS - 1) / CS);
         a.dx_steps = (nsteps + S - 1) / S;

@@ -163,6 +163,9 @@ int launch_split_reduce(const float *part, int S, int64_t M, int64_t N, const Ou
 // Prefill (more than 64 rows) dequant-matmul on 32x32x16 MFMA (prefill.hip).
 int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDesc &y, void *ws,
                    size_t ws_bytes, hipStream_t stream);
+// rexp[m] = row_exponent(max |x[m]|) and xh[m][k] = fp16(x[m][k] * 2^-rexp[m]),
+// xh [M][K] (prefill.hip): K % 8 == 0, x's rows 16-byte aligned.
+int launch_row_prep(const ActDesc &x, int64_t M, int64_t K, int *rexp, void *xh, hipStream_t stream);
 bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M);
 size_t prefill_workspace(int64_t M, int64_t N, int64_t K, int levels);
 

@@ -35,7 +35,7 @@
 //    us against mm_kernel, 6144 x 2048 at M = 2048 131.8 -> 99.9 us (36.2 and
 //    88.4 since);
 //  * activations are converted once to fp16 after the exact per-row
-//    power-of-two rescale by a pre-kernel (pf_prep_kernel, into the
+//    power-of-two rescale by a pre-kernel (row_prep_kernel, into the
 //    workspace) and staged in LDS as they are, double buffered: step k + 1
 //    is stored while step k is multiplied;
 //  * weight loads run PD steps ahead in registers (buffer loads: a row past
@@ -102,80 +102,124 @@ struct PfArgs {
     int64_t estride_w, estride_s;
 };
 
-// Per-row exponent of the largest |x| (row_exponent), then the row rescaled
-// by 2^-e and rounded to fp16 into xh [M][K] (one wave per row, 16-byte
-// loads, four in flight per lane; the second pass re-reads the row from the
-// caches).  Converting once here saves the main kernel a conversion per
-// N tile.
-__global__ void __launch_bounds__(256)
-    pf_prep_kernel(const void *x, int xdt, int64_t ldx, int M, int K, int *rexp, f16_t *xh)
+// Pieces of 8 values of a row for row_prep_kernel.
+template <int XDT>
+EP_DEV void prep_load(const char *base, int q, u32x4_t (&v)[XDT == EP_F32 ? 2 : 1])
 {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= M)
-        return;
-    const int esz = xdt == EP_F32 ? 4 : 2;
-    const int pieces = K * esz / 16;
-    const char *base = (const char *)x + (int64_t)row * ldx * esz;
-    float amax = 0.0f;
-    for (int p0 = lane; p0 < pieces; p0 += 256) {
-        u32x4_t v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int p = p0 + 64 * u;
-            v[u] = p < pieces ? *(const __attribute__((address_space(1))) u32x4_t *)(base + (int64_t)p * 16)
-                              : (u32x4_t){0u, 0u, 0u, 0u};
+    for (int i = 0; i < (XDT == EP_F32 ? 2 : 1); ++i)
+        v[i] = *(const __attribute__((address_space(1))) u32x4_t *)(base + (int64_t)q * (XDT == EP_F32 ? 32 : 16) +
+                                                                   16 * i);
+}
+
+template <int XDT>
+EP_DEV void prep_values(const u32x4_t (&r)[XDT == EP_F32 ? 2 : 1], float (&v)[8])
+{
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        if constexpr (XDT == EP_F32) {
+            v[t] = __uint_as_float(r[0][t]);
+            v[4 + t] = __uint_as_float(r[1][t]);
+        } else {
+            unpack_pair<XDT>(r[0][t], v[2 * t], v[2 * t + 1]);
         }
+    }
+}
+
+template <int XDT>
+EP_DEV float prep_max(const u32x4_t (&r)[XDT == EP_F32 ? 2 : 1], float amax)
+{
+    float v[8];
+    prep_values<XDT>(r, v);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int t = 0; t < 8; ++t)
+        amax = fmaxf(amax, fabsf(v[t]));
+    return amax;
+}
+
+template <int XDT>
+EP_DEV f16x8_t prep_round(const u32x4_t (&r)[XDT == EP_F32 ? 2 : 1], float pw)
+{
+    float v[8];
+    prep_values<XDT>(r, v);
+    f16x8_t h;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const uint32_t r = v[u][t];
-                if (xdt == EP_F32) {
-                    amax = fmaxf(amax, fabsf(__uint_as_float(r)));
-                } else {
-                    float lo, hi;
-                    if (xdt == EP_BF16)
-                        unpack_pair<EP_BF16>(r, lo, hi);
-                    else
-                        unpack_pair<EP_F16>(r, lo, hi);
-                    amax = fmaxf(amax, fmaxf(fabsf(lo), fabsf(hi)));
-                }
-            }
+    for (int t = 0; t < 8; ++t)
+        h[t] = (f16_t)(v[t] * pw);
+    return h;
+}
+
+// Per-row exponent of the largest |x| (row_exponent), then the row rescaled
+// by 2^-e and rounded to fp16 into xh [M][K]: converting once here saves the
+// main kernel a conversion per N tile.  Bound by the latency of a row's
+// loads, not by their bytes: a workgroup takes one row and each thread holds
+// its PP pieces of 8 values in registers from the maximum to the rescale (a
+// wave per row read the row twice, in a chain of loads and waits).
+// bf16 rows: 201 x 6144 8.9 -> 3.3 us, 4096 x 2048 9.3 -> 7.3, 2048 x 2048
+// 6.4 -> 5.4.
+// Pieces past the row's end are clamped to its last one; those of rows
+// beyond 8 pieces per thread are read again for the rescale.
+template <int XDT, int PP>
+__global__ void __launch_bounds__(256) row_prep_kernel(const void *x, int64_t ldx, int K, int *rexp, f16_t *xh)
+{
+    __shared__ float s_max[4];
+    const int tid = threadIdx.x, nt = blockDim.x, row = blockIdx.x;
+    const int pieces = K / 8;
+    const char *base = (const char *)x + (int64_t)row * ldx * (XDT == EP_F32 ? 4 : 2);
+    u32x4_t v[PP][XDT == EP_F32 ? 2 : 1];
+#pragma unroll
+    for (int p = 0; p < PP; ++p)
+        prep_load<XDT>(base, min(tid + p * nt, pieces - 1), v[p]);
+    float amax = 0.0f;
+#pragma unroll
+    for (int p = 0; p < PP; ++p)
+        amax = prep_max<XDT>(v[p], amax);
+    for (int q = tid + PP * nt; q < pieces; q += nt) {
+        u32x4_t r[XDT == EP_F32 ? 2 : 1];
+        prep_load<XDT>(base, q, r);
+        amax = prep_max<XDT>(r, amax);
     }
     amax = wave_max(amax);
+    if (nt > 64) {  // uniform
+        if ((tid & 63) == 0)
+            s_max[tid >> 6] = amax;
+        __syncthreads();
+        for (int w = 0; w < nt / 64; ++w)
+            amax = fmaxf(amax, s_max[w]);
+    }
     const int e = row_exponent(amax);
-    if (lane == 0)
+    if (tid == 0)
         rexp[row] = e;
     const float pw = ldexpf(1.0f, -e);
-    // output pieces of 8 values: 16 input bytes (2-byte types) or 32 (f32)
     f16x8_t *dst = (f16x8_t *)(xh + (int64_t)row * K);
-    for (int q = lane; q < K / 8; q += 64) {
-        float v[8];
-        if (xdt == EP_F32) {
-            const u32x4_t a0 = *(const __attribute__((address_space(1))) u32x4_t *)(base + (int64_t)q * 32);
-            const u32x4_t a1 = *(const __attribute__((address_space(1))) u32x4_t *)(base + (int64_t)q * 32 + 16);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                v[t] = __uint_as_float(a0[t]);
-                v[4 + t] = __uint_as_float(a1[t]);
-            }
-        } else {
-            const u32x4_t a0 = *(const __attribute__((address_space(1))) u32x4_t *)(base + (int64_t)q * 16);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                if (xdt == EP_BF16)
-                    unpack_pair<EP_BF16>(a0[t], v[2 * t], v[2 * t + 1]);
-                else
-                    unpack_pair<EP_F16>(a0[t], v[2 * t], v[2 * t + 1]);
-            }
-        }
-        f16x8_t h;
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-            h[t] = (f16_t)(v[t] * pw);
-        dst[q] = h;
+    for (int p = 0; p < PP; ++p)
+        if (tid + p * nt < pieces)
+            dst[tid + p * nt] = prep_round<XDT>(v[p], pw);
+    for (int q = tid + PP * nt; q < pieces; q += nt) {
+        u32x4_t r[XDT == EP_F32 ? 2 : 1];
+        prep_load<XDT>(base, q, r);
+        dst[q] = prep_round<XDT>(r, pw);
     }
+}
+
+template <int XDT>
+void row_prep_x(const void *x, int64_t ldx, int64_t M, int64_t K, int *rexp, f16_t *xh, hipStream_t stream)
+{
+    // as many waves (up to four) as the row has 64 pieces, then as few
+    // pieces per thread as cover it
+    const int64_t pieces = K / 8;
+    const int nt = pieces <= 64 ? 64 : (pieces <= 128 ? 128 : 256);
+    const int64_t pp = (pieces + nt - 1) / nt;
+    const dim3 grid((unsigned)M), block((unsigned)nt);
+    if (pp <= 1)
+        hipLaunchKernelGGL((row_prep_kernel<XDT, 1>), grid, block, 0, stream, x, ldx, (int)K, rexp, xh);
+    else if (pp <= 2)
+        hipLaunchKernelGGL((row_prep_kernel<XDT, 2>), grid, block, 0, stream, x, ldx, (int)K, rexp, xh);
+    else if (pp <= 4)
+        hipLaunchKernelGGL((row_prep_kernel<XDT, 4>), grid, block, 0, stream, x, ldx, (int)K, rexp, xh);
+    else
+        hipLaunchKernelGGL((row_prep_kernel<XDT, 8>), grid, block, 0, stream, x, ldx, (int)K, rexp, xh);
 }
 
 template <int BITS, int BM, int PD, int NT, int WAVES, bool GR, bool SF32, bool G128>
@@ -184,7 +228,7 @@ __global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
     constexpr int SB = SF32 ? 4 : 2;             // bytes of a group scale
     constexpr int MT = BM / 32;                  // 32-row M tiles per wave
     constexpr int THREADS = WAVES * 64;
-    constexpr int XE = 2;  // activations: fp16, pre-scaled per row (pf_prep_kernel)
+    constexpr int XE = 2;  // activations: fp16, pre-scaled per row (row_prep_kernel)
     constexpr int XROWS = THREADS / 8;           // activation rows per staging load (8 threads a row)
     constexpr int XP = BM / XROWS;               // 16-byte pieces per staging thread and step
     constexpr int WL = BITS == 4 ? 1 : 2;        // 16-byte weight loads per lane, N tile and step
@@ -628,9 +672,8 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     const bool sf32 = w.scale_dtype == EP_F32;
     int *rexp = (int *)ws;
     f16_t *xh = (f16_t *)((char *)ws + (T * 4 + 255) / 256 * 256);
-    hipLaunchKernelGGL(pf_prep_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, stream, x.ptr, x.dtype,
-                       x.ld, (int)T, (int)w.K, rexp, xh);
-    EP_HIP_CHECK(hipGetLastError());
+    if (const int rc = launch_row_prep(x, T, w.K, rexp, xh, stream); rc != EP_OK)
+        return rc;
     PfArgs a{};
     a.xbytes = (uint32_t)(T * w.K * 2);
     a.wbytes = (uint32_t)(w.N * (bits == 4 ? w.K / 2 : w.K));
@@ -682,6 +725,18 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     return pf_launch_grouped<8, 64, 4, 2, 4>(a, tiles_y, sf32, stream);
 }
 
+int launch_row_prep(const ActDesc &x, int64_t M, int64_t K, int *rexp, void *xh, hipStream_t stream)
+{
+    if (x.dtype == EP_F32)
+        row_prep_x<EP_F32>(x.ptr, x.ld, M, K, rexp, (f16_t *)xh, stream);
+    else if (x.dtype == EP_F16)
+        row_prep_x<EP_F16>(x.ptr, x.ld, M, K, rexp, (f16_t *)xh, stream);
+    else
+        row_prep_x<EP_BF16>(x.ptr, x.ld, M, K, rexp, (f16_t *)xh, stream);
+    EP_HIP_CHECK(hipGetLastError());
+    return EP_OK;
+}
+
 bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
 {
     const int bits = w.bits();
@@ -728,9 +783,8 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
         return set_error(EP_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, ws_bytes);
     int *rexp = (int *)ws;
     f16_t *xh = (f16_t *)((char *)ws + ex);
-    hipLaunchKernelGGL(pf_prep_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, stream, x.ptr, x.dtype,
-                       x.ld, (int)M, (int)w.K, rexp, xh);
-    EP_HIP_CHECK(hipGetLastError());
+    if (const int rc = launch_row_prep(x, M, w.K, rexp, xh, stream); rc != EP_OK)
+        return rc;
     PfArgs a{};
     a.xbytes = (uint32_t)(M * w.K * 2);
     a.wbytes = (uint32_t)(w.N * (bits == 4 ? w.K / 2 : w.K));

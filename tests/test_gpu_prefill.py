@@ -210,3 +210,26 @@ def test_f32_scales_on_the_tiles(levels, group, m, n, k):
     _, x = x_bf16(m, k, m)
     want = (x.double() @ s.materialize(torch.float16).double().t()).cpu().numpy()
     assert_close(run(s, x).cpu().numpy(), want, 1e-4)
+
+
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k", [64, 512, 576, 1024, 1088, 2112, 4160, 8256, 16384, 16448])
+def test_row_prep_row_lengths(k, xdt):
+    """The row exponents and fp16 activations at row lengths on either side of
+    every split of a row over threads (64 / 128 / 256 threads, 1 / 2 / 4 / 8
+    pieces each, and pieces past 8), from a view with a longer row stride,
+    each row's largest value in another place.  Against the f64 product of x
+    and the fp16 weights: fp16 rounds each x to 2^-11 of itself at most,
+    independently, so a row's sums move by about 2^-11 of their own rms (K
+    terms on both sides), and their largest deviation of 128 by less than
+    four times that, against the largest of the row."""
+    m, n = 70, 128
+    _, packed, scale, cb, s = make(n, k, 16, 64, seed=k)
+    x32 = rng(k + 1).standard_normal((m, k + 8)).astype(np.float32)
+    x32 *= np.exp2(rng(k + 2).integers(-12, 8, (m, 1))).astype(np.float32)
+    x32[np.arange(m), (np.arange(m) * 977) % k] *= 64.0
+    x = torch.from_numpy(x32).to(DEV).to(xdt)[:, :k]
+    want = (x.double() @ s.materialize(torch.float16).double().t()).cpu().numpy()
+    y = run(s, x).double().cpu().numpy()
+    rows = np.abs(want).max(1, keepdims=True)
+    assert (np.abs(y - want) / rows).max() <= 4 * 2.0 ** -11
