@@ -276,3 +276,21 @@ def test_backward_library_route_many_token_counts():
     x, gy = first[0], first[1]
     again = run_bwd(s, gy, x)
     assert all(torch.equal(p, q) for p, q in zip(first[2:], again))
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("n,k,m", [(16, 128, 1), (144, 256, 63), (272, 384, 65), (2064, 2176, 129),
+                                   (6160, 256, 520)])
+def test_gradient_reductions_at_tile_edges(group, n, k, m):
+    """grad_scale and grad_cb where the last weight tile has 16 rows, tokens
+    end one before and after a step, and the per-workgroup codebook sums are
+    1, a few, more than 256 and more than 2048 (6160 rows: the library route),
+    for every number of groups per tile.  f32 sums of exact bf16 products:
+    at most (m + n k / 16) * 2^-24 of the sum of magnitudes; held to 1e-4 of
+    the largest."""
+    _, _, _, _, s = make(n, k, group, seed=n + group)
+    x, gy = bf16((m, k), 3), bf16((m, n), 4, 1e-2)
+    _, gcb, gsc = run_bwd(s, gy, x)
+    _, wcb, wsc = closed_forms_t64(gy, x, s)
+    assert rel(gsc, wsc) < 1e-4
+    assert rel(gcb, wcb) < 1e-4
