@@ -90,65 +90,70 @@ __global__ void __launch_bounds__(256) dequant_tile_kernel(TileArgs a)
 }
 
 // The same tile for 4-bit rows of whole 16-byte chunks (K % 32 == 0, groups
-// of 32·2^i): one thread per 16 packed bytes (32 weights, one group scale),
-// the codebook pre-rounded in LDS, 16-byte stores.  Same arithmetic as
-// dequant_elem (round(c) * round(s) in fp32, rounded once).
-constexpr int kTile4 = 1;
+// of a multiple of 32), bound by its stores: a wave takes one row, a lane 4
+// packed bytes (8 weights, one group scale) of each 512, four loads in
+// flight, so a store instruction writes 1 KiB (2-byte types) in one piece.
+// A thread per 32 weights, its four stores 64 bytes from its neighbours',
+// took twice as long: 6144 x 2048
+// to fp16 beside the backward's other product 23.8 -> 11.3 us.  The codebook is pre-rounded in LDS.  Same arithmetic as dequant_elem (round(c) * round(s) in fp32,
+// rounded once).
+constexpr int kTile4 = 4;  // loads in flight per lane
 template <int DT>
 __global__ void __launch_bounds__(256) dequant_tile4_kernel(TileArgs a)
 {
     __shared__ float tab[16];
+    const int lane = threadIdx.x & 63;
+    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t row = n < a.N ? n : a.N - 1;  // every wave reaches the barrier
+    const int dw = (int)(a.K / 8);
+    const uint32_t *src = (const uint32_t *)(a.packed + row * (a.K / 2));
+    char *dst = (char *)a.out + row * a.ldo * (DT == EP_F32 ? 4 : 2);
+    uint32_t w[kTile4];
+    float sc[kTile4];
+    auto load = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < kTile4; ++u) {
+            const int i = min(i0 + 64 * u, dw - 1);
+            w[u] = src[i];
+            sc[u] = load_as_f32(a.scale, a.scale_dtype, row * a.lds + (uint32_t)i * 8u / (uint32_t)a.group);
+        }
+    };
+    load(lane);
     if (threadIdx.x < 16)
         tab[threadIdx.x] = threadIdx.x < a.levels ? round_to(DT, load_as_f32(a.cb, a.cb_dtype, threadIdx.x)) : 0.0f;
-    __syncthreads();
-    const int64_t cpr = a.K / 32;  // chunks per row
-    const int64_t total = a.N * cpr;
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    // kTile4 chunks per thread, all loaded before the first is expanded
-    u32x4_t wv[kTile4];
-    float scv[kTile4];
+    lds_barrier();
+    if (n >= a.N)
+        return;
+    for (int i0 = lane; i0 < dw; i0 += 64 * kTile4) {
 #pragma unroll
-    for (int j = 0; j < kTile4; ++j) {
-        const int64_t i = i0 + j * stride < total ? i0 + j * stride : 0;
-        const int64_t n = i / cpr, c = i % cpr;
-        wv[j] = *(const u32x4_t *)(a.packed + n * (a.K / 2) + c * 16);
-        scv[j] = load_as_f32(a.scale, a.scale_dtype, n * a.lds + (c * 32) / a.group);
-    }
+        for (int u = 0; u < kTile4; ++u) {
+            const int i = i0 + 64 * u;
+            if (i >= dw)
+                break;
+            const float s = round_to(DT, sc[u]);
+            float v[8];
 #pragma unroll
-    for (int j = 0; j < kTile4; ++j) {
-    const int64_t i = i0 + j * stride;
-    if (i >= total)
-        break;
-    const int64_t n = i / cpr, c = i % cpr;
-    const u32x4_t w = wv[j];
-    const float sc = round_to(DT, scv[j]);
-    float v[32];
+            for (int t = 0; t < 8; ++t)
+                v[t] = tab[(w[u] >> (4 * t)) & 15] * s;
+            if constexpr (DT == EP_F32) {
+                f32x4_t *d = (f32x4_t *)dst + (int64_t)i * 2;
+                d[0] = (f32x4_t){v[0], v[1], v[2], v[3]};
+                d[1] = (f32x4_t){v[4], v[5], v[6], v[7]};
+            } else {
+                u32x4_t o;
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-            v[d * 8 + t] = tab[(w[d] >> (4 * t)) & 15] * sc;
-    char *dst = (char *)a.out + (n * a.ldo + c * 32) * (DT == EP_F32 ? 4 : 2);
-    if constexpr (DT == EP_F32) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-            ((f32x4_t *)dst)[q] = (f32x4_t){v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            u32x4_t o;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float lo = v[8 * q + 2 * t], hi = v[8 * q + 2 * t + 1];
-                if constexpr (DT == EP_F16)
-                    o[t] = (uint32_t)f16_bits((f16_t)lo) | ((uint32_t)f16_bits((f16_t)hi) << 16);
-                else
-                    o[t] = (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
+                for (int t = 0; t < 4; ++t) {
+                    const float lo = v[2 * t], hi = v[2 * t + 1];
+                    if constexpr (DT == EP_F16)
+                        o[t] = (uint32_t)f16_bits((f16_t)lo) | ((uint32_t)f16_bits((f16_t)hi) << 16);
+                    else
+                        o[t] = (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
+                }
+                ((u32x4_t *)dst)[i] = o;
             }
-            ((u32x4_t *)dst)[q] = o;
         }
-    }
+        if (i0 + 64 * kTile4 < dw)
+            load(i0 + 64 * kTile4);
     }
 }
 
@@ -191,10 +196,10 @@ int launch_dequant_tile(const PackedDesc &w, void *out, int out_dtype, int64_t l
     const int esz = out_dtype == EP_F32 ? 4 : 2;
     const bool fast = w.levels <= 16 && w.K % 32 == 0 && w.group % 32 == 0 &&
                       ((uintptr_t)w.packed & 15) == 0 && ((uintptr_t)out & 15) == 0 &&
-                      (ldo * esz) % 16 == 0 && (w.N * (w.K / 32) + 255) / 256 < 0x7fffffff &&
-                      w.N * (w.K / 32) >= 1;
+                      (ldo * esz) % 16 == 0 && w.K <= 0x7fffffff &&
+                      w.N <= 0x7fffffff;
     if (fast) {
-        const dim3 grid((unsigned)((w.N * (w.K / 32) + 256 * kTile4 - 1) / (256 * kTile4)));
+        const dim3 grid((unsigned)((w.N + 3) / 4));
         if (out_dtype == EP_F16)
             hipLaunchKernelGGL(dequant_tile4_kernel<EP_F16>, grid, dim3(256), 0, stream, a);
         else if (out_dtype == EP_BF16)

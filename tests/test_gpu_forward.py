@@ -106,6 +106,19 @@ def test_dequant_tile_bitexact(dtype, name, levels, n, k, group):
     assert np.array_equal(w, want)
 
 
+@pytest.mark.parametrize("dtype,name", [(torch.float32, "f32"), (torch.float16, "f16"),
+                                        (torch.bfloat16, "bf16")])
+@pytest.mark.parametrize("n,k,group", [(1, 32, 32), (3, 480, 32), (4, 512, 64), (5, 544, 32),
+                                       (6, 2048, 128), (9, 2080, 32), (2, 14336, 96)])
+def test_dequant_rows_bitexact(dtype, name, n, k, group):
+    """4-bit rows of whole 16-byte chunks at lengths around a wave's 512
+    weights and its 2048 in flight, and rows around four per workgroup."""
+    _, packed, scale, cb = ref.synth_linear(n, k, 16, group, seed=n + k)
+    s = PackedWeight((n, k), packed, scale, cb.astype(np.float32), group, 16).to(DEV)
+    w = s.materialize(dtype).float().cpu().numpy()
+    assert np.array_equal(w, ref.materialize(packed, scale, cb.astype(np.float32), n, k, group, 16, name))
+
+
 # ------------------------------------------------------------------ batch-1 GEMV
 def test_gemv_config0_shape():
     n = k = 4096
