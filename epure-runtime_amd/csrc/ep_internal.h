@@ -148,7 +148,7 @@ int launch_expert_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, cons
 bool prefill_grouped_serves(const PackedDesc &w, const ActDesc &x, int64_t T);
 size_t prefill_grouped_workspace(int64_t T, int64_t K);
 int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, const int *perm,
-                           const int *tiles, const int *ntiles, int bm, unsigned tiles_y, const OutDesc &y,
+                           const int *tiles, const int *ntiles, int64_t experts, int bm, unsigned tiles_y, const OutDesc &y,
                            void *ws, hipStream_t stream);
 
 // Small-M (2..64 rows) split-K dequant-matmul on MFMA (skinny.hip).

@@ -607,7 +607,7 @@ int launch_expert_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, cons
     EP_HIP_CHECK(hipGetLastError());
     const unsigned ty = (unsigned)grouped_max_tiles(T, E, bm);
     if (pf)
-        return launch_prefill_grouped(w, x, T, perm, tiles, ntiles, bm, ty, y, rexp, stream);
+        return launch_prefill_grouped(w, x, T, perm, tiles, ntiles, E, bm, ty, y, rexp, stream);
     const dim3 rg((unsigned)((T + 3) / 4));
     if (x.dtype == EP_BF16)
         hipLaunchKernelGGL(row_exp16_kernel<EP_BF16>, rg, dim3(256), 0, stream, x.ptr, x.ld, (int)T, w.K, rexp);

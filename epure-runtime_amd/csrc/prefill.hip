@@ -19,7 +19,8 @@
 //    CU keeps ~32 KiB of loads in flight), so wider workgroups -- more weight
 //    rows per staged activation tile -- measured faster than 4-wave ones
 //    (8-bit 1.1-1.15x) and than two weight tiles at 64 activation rows
-//    (8-bit 1.25x); smaller M runs 4 waves x BM = 64 x two tiles;
+//    (8-bit 1.25x); smaller M runs 8 waves x BM = 64 x one tile, two
+//    workgroups per CU (M <= 32: 4 waves x 32 rows x two tiles);
 //  * lane (j = lane & 31, h = lane >> 5) of a wave holds, per 64-k step and
 //    N tile, 32 consecutive weights of row j (k = 32 h .. 32 h + 31 of the
 //    step: one 16-byte load at 4 bits, two at 8 bits); MFMA sub-step s takes
@@ -587,28 +588,23 @@ struct PfPlan {
 PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
 {
     PfPlan p;
-    if (bits == 4) {
-        // measured: 128 x 2 tiles lead from M = 1024, 128 x 1 at 256..1023
-        p.bm = M >= EP_PF_BIG4_M ? 128 : M > 32 ? 64 : 32;
-        p.nt = M >= EP_PF_BIG4_M && M < 1024 ? 1 : 2;
-        p.waves = M >= EP_PF_BIG4_M ? 8 : 4;
-    } else if (M >= EP_PF_BIG8_M) {
-        p.bm = 128;
-        p.nt = 1;
-        p.waves = 8;
-    } else {
-        p.bm = M > 32 ? 64 : 32;
-        p.nt = 2;
-        p.waves = 4;
-    }
+    // measured: 128 x 2 tiles lead from M = 1024 (4-bit), 128 x 1 below.  The
+    // 64-row tile on eight waves of one weight tile, two workgroups per CU
+    // (four waves of two left a SIMD two waves to hide a step's lookups and
+    // loads behind): 4-bit 4096^2 at M = 100 28.2 -> 24.3 us a call, 8192 x
+    // 4096 at 65 31.6 -> 28.9, 8-bit 4096 x 14336 at 100 46.0 -> 40.3, 14336 x
+    // 4096 at 127 48.1 -> 44.6.
+    p.bm = M >= (bits == 4 ? EP_PF_BIG4_M : EP_PF_BIG8_M) ? 128 : M > 32 ? 64 : 32;
+    p.nt = p.bm == 32 || (p.bm == 128 && bits == 4 && M >= 1024) ? 2 : 1;
+    p.waves = p.bm == 32 ? 4 : 8;
     const int bn = p.waves * 32 * p.nt;
     const int64_t tiles = ((N + bn - 1) / bn) * ((M + p.bm - 1) / p.bm);
     const int nk = (int)(K / kPfBK);
     // K split in two while the grid stays within one round of resident
-    // workgroups (8 waves per CU): a split past that only adds partials
-    // (14336 x 4096 at M = 512, 224 tiles: 132.7 us with 2 splits, 110.5
+    // workgroups (one per CU at 128 rows, else two): a split past that only
+    // adds partials (14336 x 4096 at M = 512, 224 tiles: 132.7 us with 2 splits, 110.5
     // with none; M = 256, 112 tiles: 93.6 us with 4, 80.9 with 2)
-    const int target = 8 / p.waves * device_cus();
+    const int target = (p.bm == 128 ? 1 : 2) * device_cus();
     int S = 1;
     while (tiles * S * 2 <= target && S < 8 && nk / (S * 2) >= 8)
         S *= 2;
@@ -665,8 +661,8 @@ size_t prefill_grouped_workspace(int64_t T, int64_t K)
 // copy of every token row, then pf_kernel over each expert's row tiles (bm
 // 64 or 128 rows, the whole K per workgroup), results at the tokens' rows.
 int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, const int *perm,
-                           const int *tiles, const int *ntiles, int bm, unsigned tiles_y, const OutDesc &y,
-                           void *ws, hipStream_t stream)
+                           const int *tiles, const int *ntiles, int64_t experts, int bm, unsigned tiles_y,
+                           const OutDesc &y, void *ws, hipStream_t stream)
 {
     const int bits = w.bits();
     const bool sf32 = w.scale_dtype == EP_F32;
@@ -709,20 +705,33 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     a.estride_w = w.N * (int64_t)a.row_bytes;
     a.estride_s = w.N * w.ld_scale;
     a.ksteps = (nk + 1) / 2 * 2;  // the whole K per workgroup
+    // 64-row tiles: one 32-row weight tile per wave, so that a SIMD has four
+    // waves to hide a step's lookups and loads behind (four waves of two
+    // tiles left it two); eight waves, or four (128 weight rows) where those
+    // workgroups, two per CU, are all resident at the experts' mean rows.
+    // Whole calls, 4-bit: 128 x 768 x 2048, 4096 rows, four waves of two
+    // tiles / eight / four of one: 73.8 / 67.9 / 72.8 us; 64 x 2048 x 1024
+    // 85.4 / 71.0 / 78.2; 8 x 2048 x 3072, 300 rows 52.2 / 44.1 / 38.5; 8-bit
+    // 128 x 768 x 2048 92.3 / 83.7 / 81.7; 32 x 1024 x 2048, 1200 rows 60.7 /
+    // 49.6 / 43.1.
+    const int64_t mean = (T + experts - 1) / experts;
+    const bool narrow = experts * ((mean + 63) / 64) * ((w.N + 127) / 128) <= 2 * (int64_t)device_cus();
     if (bits == 4) {
         if (bm == 128) {
             return pf_launch_grouped<4, 128, 4, 1, 8>(a, tiles_y, sf32, stream);
         }
         if (bm == 32)
             return pf_launch_grouped<4, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
-        return pf_launch_grouped<4, 64, 4, 2, 4>(a, tiles_y, sf32, stream);
+        return narrow ? pf_launch_grouped<4, 64, 4, 1, 4>(a, tiles_y, sf32, stream)
+                      : pf_launch_grouped<4, 64, 4, 1, 8>(a, tiles_y, sf32, stream);
     }
     if (bm == 128) {
         return pf_launch_grouped<8, 128, EP_PF_PD8, 1, 8>(a, tiles_y, sf32, stream);
     }
     if (bm == 32)
         return pf_launch_grouped<8, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
-    return pf_launch_grouped<8, 64, 4, 2, 4>(a, tiles_y, sf32, stream);
+    return narrow ? pf_launch_grouped<8, 64, 4, 1, 4>(a, tiles_y, sf32, stream)
+                  : pf_launch_grouped<8, 64, 4, 1, 8>(a, tiles_y, sf32, stream);
 }
 
 int launch_row_prep(const ActDesc &x, int64_t M, int64_t K, int *rexp, void *xh, hipStream_t stream)
@@ -816,13 +825,13 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
     a.part = partials ? (float *)((char *)ws + ex + xhb) : nullptr;
     int rc;
     if (bits == 4)
-        rc = p.nt == 1 ? pf_launch<4, 128, 4, 1, 8>(a, p, sf32, stream)
-             : p.bm == 128 ? pf_launch<4, 128, 2, 2, 8>(a, p, sf32, stream)
-             : p.bm == 64  ? pf_launch<4, 64, 4, 2, 4>(a, p, sf32, stream)
-                           : pf_launch<4, 32, 4, 2, 4>(a, p, sf32, stream);
+        rc = p.bm == 128  ? (p.nt == 1 ? pf_launch<4, 128, 4, 1, 8>(a, p, sf32, stream)
+                                       : pf_launch<4, 128, 2, 2, 8>(a, p, sf32, stream))
+             : p.bm == 64 ? pf_launch<4, 64, 4, 1, 8>(a, p, sf32, stream)
+                          : pf_launch<4, 32, 4, 2, 4>(a, p, sf32, stream);
     else
-        rc = p.nt == 1   ? pf_launch<8, 128, EP_PF_PD8, 1, 8>(a, p, sf32, stream)
-             : p.bm == 64 ? pf_launch<8, 64, 4, 2, 4>(a, p, sf32, stream)
+        rc = p.bm == 128  ? pf_launch<8, 128, EP_PF_PD8, 1, 8>(a, p, sf32, stream)
+             : p.bm == 64 ? pf_launch<8, 64, 4, 1, 8>(a, p, sf32, stream)
                           : pf_launch<8, 32, 4, 2, 4>(a, p, sf32, stream);
     if (rc != EP_OK || !partials)
         return rc;

@@ -93,10 +93,10 @@ __global__ void __launch_bounds__(256) dequant_tile_kernel(TileArgs a)
 // of a multiple of 32), bound by its stores: a wave takes one row, a lane 4
 // packed bytes (8 weights, one group scale) of each 512, four loads in
 // flight, so a store instruction writes 1 KiB (2-byte types) in one piece.
-// A thread per 32 weights, its four stores 64 bytes from its neighbours',
-// took twice as long: 6144 x 2048
-// to fp16 beside the backward's other product 23.8 -> 11.3 us.  The codebook is pre-rounded in LDS.  Same arithmetic as dequant_elem (round(c) * round(s) in fp32,
-// rounded once).
+// With a thread per 32 weights its four stores lay 64 bytes from its
+// neighbours': 6144 x 2048 to fp16 beside the backward's other product 23.8
+// us, 11 to 17 now.  The codebook is pre-rounded in LDS.  Same arithmetic as
+// dequant_elem (round(c) * round(s) in fp32, rounded once).
 constexpr int kTile4 = 4;  // loads in flight per lane
 template <int DT>
 __global__ void __launch_bounds__(256) dequant_tile4_kernel(TileArgs a)

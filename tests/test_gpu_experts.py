@@ -336,3 +336,25 @@ def test_grouped_experts_clamp_ids_and_strided_rows():
     assert torch.equal(PackedExperts(s)(x, ids), want)
     with pytest.raises(IndexError):
         PackedExperts(s)(x, bad)
+
+
+@pytest.mark.parametrize("levels", [16, 256])
+@pytest.mark.parametrize("E,n,k,T", [(3, 130, 128, 100), (3, 515, 1088, 330), (40, 1700, 192, 1300),
+                                     (40, 1665, 128, 4000)])
+def test_grouped_64_row_tiles(levels, E, n, k, T):
+    """Experts of 32 to 127 mean rows (64-row tiles) on both sides of the
+    workgroup width's rule (few weight rows in all: 128 per workgroup, else
+    256), rows of a run ending inside a tile and N inside a workgroup, against
+    the f64 product of the operands: fp16 x as it is and fp16 weights, so what
+    is left is the f32 sums (K <= 1088 products, at most 1088 * 2^-24 = 6.5e-5
+    of their magnitudes) and the fp16 output's 2^-11."""
+    s, packed, scale, cb = experts(E, n, k, levels, 64, seed=E + n)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, k, generator=g, device=DEV).to(torch.float16)
+    ids = torch.randint(0, E, (T,), generator=g, device=DEV)
+    y = PackedExperts(s)(x, ids).double()
+    w = s.materialize(torch.float16).double().view(E, n, k)
+    for e in range(E):
+        rows = (ids == e).nonzero().reshape(-1)
+        want = x[rows].double() @ w[e].t()
+        assert (y[rows] - want).abs().max() <= (2.0 ** -11 + 1e-4) * want.abs().max()
