@@ -713,15 +713,20 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
     // tiles / eight / four of one: 73.8 / 67.9 / 72.8 us; 64 x 2048 x 1024
     // 85.4 / 71.0 / 78.2; 8 x 2048 x 3072, 300 rows 52.2 / 44.1 / 38.5; 8-bit
     // 128 x 768 x 2048 92.3 / 83.7 / 81.7; 32 x 1024 x 2048, 1200 rows 60.7 /
-    // 49.6 / 43.1.
+    // 49.6 / 43.1.  32-row tiles take four waves: of one weight tile by the
+    // same rule (4-bit 8 x 2048 x 3072, 120 rows 43.8 -> 33.7 us; past it two
+    // stay ahead: 128 x 1536 x 2048, 3200 rows 99.3 against 102.0), and with
+    // 8-bit indices, a lookup per weight, always (32 x 1024 x 2048, 400 rows
+    // 50.8 -> 36.8; 128 x 768 x 2048, 1024 rows 69.2 -> 64.6).
     const int64_t mean = (T + experts - 1) / experts;
-    const bool narrow = experts * ((mean + 63) / 64) * ((w.N + 127) / 128) <= 2 * (int64_t)device_cus();
+    const bool narrow = experts * ((mean + bm - 1) / bm) * ((w.N + 127) / 128) <= 2 * (int64_t)device_cus();
     if (bits == 4) {
         if (bm == 128) {
             return pf_launch_grouped<4, 128, 4, 1, 8>(a, tiles_y, sf32, stream);
         }
         if (bm == 32)
-            return pf_launch_grouped<4, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
+            return narrow ? pf_launch_grouped<4, 32, 4, 1, 4>(a, tiles_y, sf32, stream)
+                          : pf_launch_grouped<4, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
         return narrow ? pf_launch_grouped<4, 64, 4, 1, 4>(a, tiles_y, sf32, stream)
                       : pf_launch_grouped<4, 64, 4, 1, 8>(a, tiles_y, sf32, stream);
     }
@@ -729,7 +734,7 @@ int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, con
         return pf_launch_grouped<8, 128, EP_PF_PD8, 1, 8>(a, tiles_y, sf32, stream);
     }
     if (bm == 32)
-        return pf_launch_grouped<8, 32, 4, 2, 4>(a, tiles_y, sf32, stream);
+        return pf_launch_grouped<8, 32, 4, 1, 4>(a, tiles_y, sf32, stream);
     return narrow ? pf_launch_grouped<8, 64, 4, 1, 4>(a, tiles_y, sf32, stream)
                   : pf_launch_grouped<8, 64, 4, 1, 8>(a, tiles_y, sf32, stream);
 }

@@ -340,10 +340,10 @@ def test_grouped_experts_clamp_ids_and_strided_rows():
 
 @pytest.mark.parametrize("levels", [16, 256])
 @pytest.mark.parametrize("E,n,k,T", [(3, 130, 128, 100), (3, 515, 1088, 330), (40, 1700, 192, 1300),
-                                     (40, 1665, 128, 4000)])
-def test_grouped_64_row_tiles(levels, E, n, k, T):
-    """Experts of 32 to 127 mean rows (64-row tiles) on both sides of the
-    workgroup width's rule (few weight rows in all: 128 per workgroup, else
+                                     (40, 1665, 128, 4000), (3, 131, 320, 61), (40, 1700, 192, 900)])
+def test_grouped_row_tiles(levels, E, n, k, T):
+    """Experts of 32 to 127 mean rows (64-row tiles) and fewer (32-row tiles)
+    on both sides of the workgroup width's rule (few weight rows in all: 128 per workgroup, else
     256), rows of a run ending inside a tile and N inside a workgroup, against
     the f64 product of the operands: fp16 x as it is and fp16 weights, so what
     is left is the f32 sums (K <= 1088 products, at most 1088 * 2^-24 = 6.5e-5
