@@ -772,9 +772,12 @@ bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
     return (x.ld * esz) % 16 == 0;
 }
 
-// Workspace: row exponents, the fp16 activations, then the split partials.
+// Workspace: row exponents, the fp16 activations, then the split partials;
+// none for rows shorter than a k step, which the tiles do not serve.
 size_t prefill_workspace(int64_t M, int64_t N, int64_t K, int levels)
 {
+    if (K < kPfBK)
+        return 0;
     const PfPlan p = pf_plan(levels <= 16 ? 4 : 8, M, N, K);
     const size_t ex = (size_t)((M * 4 + 255) / 256 * 256);
     const size_t xh = (size_t)((M * K * 2 + 255) / 256 * 256);

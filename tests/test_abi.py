@@ -4,6 +4,8 @@ before any launch."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -101,6 +103,19 @@ def test_check_maps_codes(lib):
 def test_workspace_sizes(lib):
     assert lib.ep_dequant_matmul_workspace(1, 4096, 4096, 16, 128) >= 4
     assert lib.ep_dequant_matmul_workspace(512, 4096, 4096, 16, 128) >= 512 * 4
+
+
+def test_workspace_of_rows_shorter_than_a_k_step():
+    # in a child: a division by the zero step count ends the process.  What
+    # runs such rows needs the row exponents (and, at 2..64 rows, partials)
+    shapes = [(m, 64, k) for m in (1, 4, 5, 64, 65, 2048) for k in (0, 1, 32, 63)]
+    code = ("import sys, torch; sys.path.insert(0, %r); from epure.kernels import _abi; lib = _abi._load()\n"
+            "for m, n, k in %r: print(m, lib.ep_dequant_matmul_workspace(m, n, k, 16, 32), flush=True)"
+            % (os.path.join(ROOT, "epure-runtime_amd"), shapes))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+    rows = [tuple(map(int, line.split())) for line in r.stdout.splitlines()]
+    assert len(rows) == len(shapes) and all(size >= 4 * m for m, size in rows)
 
 
 # ---- persistent decode step (include/epure_decode.h): host-side contract

@@ -119,6 +119,20 @@ def test_dequant_rows_bitexact(dtype, name, n, k, group):
     assert np.array_equal(w, ref.materialize(packed, scale, cb.astype(np.float32), n, k, group, 16, name))
 
 
+@pytest.mark.parametrize("levels,n,k,group", [(16, 70, 32, 32), (256, 33, 48, 16), (16, 64, 1, 32)])
+@pytest.mark.parametrize("m", [4, 5, 64, 65])
+def test_rows_shorter_than_a_k_step(levels, n, k, group, m):
+    """K below the tiles' 64-value step: the generic kernel, and past 64 rows
+    the dense product of a declined call (weights rounded to x's type)."""
+    _, packed, scale, cb, s = make(n, k, levels, group, seed=n + m)
+    x32, x = x_bf16(m, k, m)
+    w = ref.materialize(packed, scale, cb.astype(np.float32), n, k, group, levels, "f32" if m <= 64 else "bf16")
+    want = x32.astype(np.float64) @ w.astype(np.float64).T
+    with torch.no_grad():
+        y = PackedLinear(s)(x)
+    assert_close(y.float().cpu().numpy(), want, TOL + 2.0 ** -8)
+
+
 # ------------------------------------------------------------------ batch-1 GEMV
 def test_gemv_config0_shape():
     n = k = 4096
