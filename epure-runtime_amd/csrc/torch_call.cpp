@@ -104,9 +104,11 @@ bool weight(const at::Tensor &packed, const at::Tensor &scale, const at::Tensor 
 }
 
 // The current stream of the tensor's device (nullptr and *ok false: a Python
-// error is set).
+// error is set).  A host tensor is refused here: its device index, -1, names
+// the current device's stream to torch, and the kernels would read host memory.
 void *stream_of(const at::Tensor &t, bool *ok)
 {
+    TORCH_CHECK_VALUE(t.is_cuda(), "expected a GPU tensor, but got one on ", t.device());
     PyObject *idx = PyLong_FromLong(t.get_device());
     PyObject *r = idx ? PyObject_CallOneArg(fn_stream, idx) : nullptr;
     Py_XDECREF(idx);

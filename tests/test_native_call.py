@@ -1,0 +1,27 @@
+"""The native call path from torch tensors (csrc/torch_call.cpp)."""
+import pytest
+import torch
+
+from epure import PackedWeight
+from epure.kernels import _abi, cuda
+
+
+def host_store(n=16, k=128, group=32):
+    g = torch.Generator().manual_seed(1)
+    packed = torch.randint(0, 256, (n * k // 2,), generator=g, dtype=torch.uint8)
+    scale = torch.rand(n, k // group, generator=g).half()
+    return PackedWeight((n, k), packed, scale, torch.randn(16, generator=g), group, 16)
+
+
+# ------------------------------------------------------------------ refusals (no GPU needed)
+def test_host_tensors_are_refused():
+    """The kernels would read host memory through the current device's
+    stream: refused as torch.cuda.current_stream(x.device) does."""
+    assert _abi._load() is not None, _abi.LOAD_ERROR
+    h = cuda._hot(host_store())
+    x = torch.zeros(8, h.K, dtype=torch.bfloat16)
+    gy = torch.zeros(8, h.N, dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        cuda.forward(x, h)
+    with pytest.raises(ValueError):
+        cuda.backward(gy, x, h)
