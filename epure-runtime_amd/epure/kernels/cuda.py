@@ -159,8 +159,8 @@ def linear(x, store):
         pars = own["_parameters"]
         packed, scale, cb = (bufs[a] if a in bufs else pars.get(a)
                              for a in ("packed", "scale", "cb"))
-        y = _abi.call.linear(x, packed, scale, cb, own["out_features"], own["in_features"],
-                             own["levels"], own["group"], SERVE_F32)
+        y = _abi.call.linear(x, packed, scale, cb, store.out_features, store.in_features,
+                             int(store.levels), int(store.group), SERVE_F32)
         if y is not NotImplemented:
             return y
     if not x.is_cuda:

@@ -25,3 +25,29 @@ def test_host_tensors_are_refused():
         cuda.forward(x, h)
     with pytest.raises(ValueError):
         cuda.backward(gy, x, h)
+
+
+class ModuleStore(torch.nn.Module):
+    """A store of another class: sizes as properties, a group read from JSON."""
+
+    def __init__(self, store):
+        super().__init__()
+        self.shape, self.levels, self.group = store.shape, store.levels, float(store.group)
+        for name in ("packed", "scale", "cb"):
+            self.register_buffer(name, getattr(store, name))
+
+    @property
+    def out_features(self):
+        return self.shape[0]
+
+    @property
+    def in_features(self):
+        return self.shape[1]
+
+
+def test_store_sizes_need_not_be_instance_attributes(monkeypatch):
+    """Sizes come from the store's attributes however they are defined; a
+    host x is declined after them."""
+    monkeypatch.setattr(cuda, "_AVAILABLE", True)
+    s = ModuleStore(host_store())
+    assert cuda.linear(torch.zeros(1, 128, dtype=torch.bfloat16), s) is None
