@@ -108,8 +108,9 @@ _SIGS = {
 XSRC_PLAIN, XSRC_RMSNORM, XSRC_SWIGLU = 0, 1, 2
 
 lib = None
-call = None  # the native call path (csrc/torch_call.cpp), bound to ``lib``
+call = None  # the native call path (csrc/torch_call.cpp), bound to ``lib``; None: ctypes calls serve
 LOAD_ERROR = None
+CALL_ERROR = None  # why ``call`` is None although ``lib`` is loaded
 TORCH_PATH = os.path.join(os.path.dirname(LIB_PATH), "epure_torch.so")
 
 
@@ -126,7 +127,7 @@ def _load_call(handle):
 
 
 def _load():
-    global lib, call, LOAD_ERROR
+    global lib, call, LOAD_ERROR, CALL_ERROR
     if lib is not None or LOAD_ERROR is not None:
         return lib
     try:
@@ -137,10 +138,14 @@ def _load():
             fn.argtypes = args
         if handle.ep_abi_version() != ABI_VERSION:
             raise ImportError(f"{LIB_NAME} ABI {handle.ep_abi_version()} != {ABI_VERSION}")
-        call = _load_call(handle)
         lib = handle
     except Exception as exc:                    # noqa: BLE001 - recorded and re-raised by callers
         LOAD_ERROR = exc
+        return lib
+    try:
+        call = _load_call(handle)
+    except Exception as exc:                    # noqa: BLE001 - absent, or built for another torch
+        CALL_ERROR = exc
     return lib
 
 

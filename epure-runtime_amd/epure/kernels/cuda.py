@@ -48,6 +48,12 @@ if _abi.lib is None:
             f"({type(IMPORT_ERROR).__name__}: {IMPORT_ERROR}); every packed linear will "
             "materialize. Build it with __graft_entry__.build().",
             RuntimeWarning, stacklevel=2)
+elif _abi.call is None and torch.cuda.is_available():
+    warnings.warn(
+        f"epure: {os.path.basename(_abi.TORCH_PATH)} failed to load ({type(_abi.CALL_ERROR).__name__}: "
+        f"{_abi.CALL_ERROR}); packed linears are called through ctypes, some 10 us more a call. "
+        "Build it with __graft_entry__.build().",
+        RuntimeWarning, stacklevel=2)
 
 SERVE_F32 = os.environ.get("EPURE_FUSED_F32") == "1"
 
@@ -106,6 +112,8 @@ def _hot(store):
 
 def forward(x2, h, out=None, accumulate=False):
     """Launch y = x2 @ W^T for a 2-D ``x2``.  Returns y, or None on decline."""
+    if _abi.call is None:
+        return _forward_ctypes(x2, h, out, accumulate)
     return _abi.call.matmul(x2, h.packed, h.scale, h.cb, h.N, h.levels, h.group, out, accumulate)
 
 
@@ -113,8 +121,52 @@ def backward(gy2, x2, h, need_x=True, need_cb=True, need_scale=True, gx_dtype=No
     """Fused backward; returns (grad_x, grad_cb, grad_scale) or None on decline.
 
     grad_x has ``gx_dtype`` (default: x's dtype)."""
+    if _abi.call is None:
+        return _backward_ctypes(gy2, x2, h, need_x, need_cb, need_scale, gx_dtype)
     return _abi.call.backward(gy2, x2, h.packed, h.scale, h.cb, h.N, h.levels, h.group, need_x,
                               need_cb, need_scale, _abi.dtype_code(gx_dtype or x2.dtype))
+
+
+def _forward_ctypes(x2, h, out, accumulate):
+    """``forward`` where the native call path is not loaded."""
+    M, K = x2.shape
+    stream = _abi.stream_handle(x2.device)
+    if out is None:
+        out = torch.empty((M, h.N), device=x2.device, dtype=x2.dtype)
+    ws_bytes = _abi.lib.ep_dequant_matmul_workspace(M, h.N, K, h.levels, h.group)
+    ws = torch.empty(ws_bytes, device=x2.device, dtype=torch.uint8) if ws_bytes else None
+    rc = _abi.lib.ep_dequant_matmul(
+        x2.data_ptr(), _abi.dtype_code(x2.dtype), x2.stride(0),
+        h.packed.data_ptr(), h.scale.data_ptr(), h.scale_dt, h.ld_scale,
+        h.cb.data_ptr(), h.cb_dt, h.levels, h.group, M, h.N, K,
+        out.data_ptr(), _abi.dtype_code(out.dtype), out.stride(0),
+        _abi.FLAG_ACCUMULATE if accumulate else 0,
+        ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+    return out if _abi.check(rc, "ep_dequant_matmul") else None
+
+
+def _backward_ctypes(gy2, x2, h, need_x, need_cb, need_scale, gx_dtype):
+    """``backward`` where the native call path is not loaded."""
+    M, N = gy2.shape
+    K = x2.shape[1]
+    stream = _abi.stream_handle(x2.device)
+    gx = torch.empty((M, K), device=x2.device, dtype=gx_dtype or x2.dtype) if need_x else None
+    G = (K + h.group - 1) // h.group
+    gcb = torch.empty(h.levels, device=x2.device, dtype=torch.float32) if need_cb else None
+    gsc = torch.empty((N, G), device=x2.device, dtype=torch.float32) if need_scale else None
+    ws_bytes = _abi.lib.ep_dequant_matmul_bwd_workspace(M, N, K, h.levels, h.group)
+    ws = torch.empty(ws_bytes, device=x2.device, dtype=torch.uint8) if ws_bytes else None
+    rc = _abi.lib.ep_dequant_matmul_bwd(
+        gy2.data_ptr(), _abi.dtype_code(gy2.dtype), gy2.stride(0),
+        x2.data_ptr(), _abi.dtype_code(x2.dtype), x2.stride(0),
+        h.packed.data_ptr(), h.scale.data_ptr(), h.scale_dt, h.ld_scale,
+        h.cb.data_ptr(), h.cb_dt, h.levels, h.group, M, N, K,
+        gx.data_ptr() if gx is not None else None,
+        _abi.dtype_code(gx.dtype if gx is not None else x2.dtype), K,
+        gcb.data_ptr() if gcb is not None else None,
+        gsc.data_ptr() if gsc is not None else None, G,
+        ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+    return (gx, gcb, gsc) if _abi.check(rc, "ep_dequant_matmul_bwd") else None
 
 
 class _PackedLinearFn(torch.autograd.Function):
@@ -154,7 +206,7 @@ def linear(x, store):
     # an inference call on plain tensors: all of it in one native call, which
     # reads pointers, strides and flags from the tensors of this call
     own = store.__dict__
-    bufs = own.get("_buffers")
+    bufs = own.get("_buffers") if _abi.call is not None else None
     if bufs is not None:
         pars = own["_parameters"]
         packed, scale, cb = (bufs[a] if a in bufs else pars.get(a)

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from epure import PackedWeight
+from epure import PackedLinear, PackedWeight
 from epure.kernels import _abi, cuda
 
 
@@ -51,3 +51,42 @@ def test_store_sizes_need_not_be_instance_attributes(monkeypatch):
     monkeypatch.setattr(cuda, "_AVAILABLE", True)
     s = ModuleStore(host_store())
     assert cuda.linear(torch.zeros(1, 128, dtype=torch.bfloat16), s) is None
+
+
+# ------------------------------------------------------------------ without the extension
+def test_library_serves_without_the_extension(monkeypatch):
+    """An extension that is absent, or was built for another torch, costs the
+    native call path only: the library stays loaded and is called by ctypes."""
+    def broken(handle):
+        raise ImportError("undefined symbol")
+    for name in ("lib", "call", "LOAD_ERROR", "CALL_ERROR"):
+        monkeypatch.setattr(_abi, name, None)
+    monkeypatch.setattr(_abi, "_load_call", broken)
+    assert _abi._load() is not None and _abi.LOAD_ERROR is None
+    assert _abi.call is None and isinstance(_abi.CALL_ERROR, ImportError)
+    h = cuda._hot(host_store())
+    with pytest.raises((ValueError, RuntimeError)):     # the stream of a host tensor
+        cuda.forward(torch.zeros(8, h.K, dtype=torch.bfloat16), h)
+
+
+@pytest.mark.gpu
+def test_calls_without_the_extension_are_the_same(monkeypatch):
+    dev = torch.device("cuda:0")
+    lin = PackedLinear(host_store(144, 256).to(dev))
+    h = cuda._hot(lin.store)
+    x = torch.randn(2, 12, 256, device=dev).to(torch.bfloat16)
+    x2, gy = x.view(24, 256), torch.randn(24, 144, device=dev).to(torch.bfloat16)
+
+    def results():
+        acc = torch.ones(24, 144, device=dev)
+        with torch.no_grad():
+            y = lin(x)
+        return [y, cuda.forward(x2, h), cuda.forward(x2, h, out=acc, accumulate=True),
+                *cuda.backward(gy, x2, h), cuda.backward(gy, x2, h, need_cb=False, need_scale=False,
+                                                         gx_dtype=torch.float32)[0]]
+    native = results()
+    assert _abi.call is not None, _abi.CALL_ERROR
+    monkeypatch.setattr(_abi, "call", None)
+    for a, b in zip(results(), native):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+    assert cuda.backward(gy.float(), x2, h) is None          # declined on both
