@@ -19,20 +19,15 @@
 
 #include <stdint.h>
 
+#include "epure_hip.h"
+
 namespace {
 
-typedef size_t (*WorkspaceFn)(int64_t, int64_t, int64_t, int, int);
-typedef int (*MatmulFn)(const void *, int, int64_t, const uint8_t *, const void *, int, int64_t, const void *, int,
-                        int, int, int64_t, int64_t, int64_t, void *, int, int64_t, int, void *, size_t, void *);
-typedef int (*BackwardFn)(const void *, int, int64_t, const void *, int, int64_t, const uint8_t *, const void *, int,
-                          int64_t, const void *, int, int, int, int64_t, int64_t, int64_t, void *, int, int64_t,
-                          float *, float *, int64_t, void *, size_t, void *);
-typedef const char *(*ErrorFn)();
-
-WorkspaceFn fn_ws, fn_bwd_ws;
-MatmulFn fn_matmul;
-BackwardFn fn_backward;
-ErrorFn fn_error;
+decltype(&ep_dequant_matmul_workspace) fn_ws;
+decltype(&ep_dequant_matmul) fn_matmul;
+decltype(&ep_dequant_matmul_bwd_workspace) fn_bwd_ws;
+decltype(&ep_dequant_matmul_bwd) fn_backward;
+decltype(&ep_last_error) fn_error;
 PyObject *fn_stream;  // torch._C._cuda_getCurrentRawStream
 
 // EP_F32 / EP_F16 / EP_BF16, or -1.
@@ -40,11 +35,11 @@ int dtype_code(const at::Tensor &t)
 {
     switch (t.scalar_type()) {
     case at::kFloat:
-        return 0;
+        return EP_F32;
     case at::kHalf:
-        return 1;
+        return EP_F16;
     case at::kBFloat16:
-        return 2;
+        return EP_BF16;
     default:
         return -1;
     }
@@ -143,7 +138,7 @@ PyObject *run_matmul(const at::Tensor &x2, const Weight &w, at::Tensor out, cons
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = fn_matmul(x2.const_data_ptr(), xdt, x2.stride(0), w.packed, w.scale, w.scale_dt, w.ld_scale, w.cb, w.cb_dt,
-                   w.levels, w.group, m, w.n, k, out.data_ptr(), ydt, out.stride(0), accumulate ? 1 : 0,
+                   w.levels, w.group, m, w.n, k, out.data_ptr(), ydt, out.stride(0), accumulate ? EP_FLAG_ACCUMULATE : 0,
                    need ? ws.data_ptr() : nullptr, need, stream);
     Py_END_ALLOW_THREADS
     if (rc < 0)
@@ -198,7 +193,7 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     if (c10::GradMode::is_enabled() && (x.requires_grad() || cb.requires_grad() || scale.requires_grad()))
         Py_RETURN_NOTIMPLEMENTED;
     const int xdt = dtype_code(x);
-    if (xdt < 0 || (xdt == 0 && !f32))
+    if (xdt < 0 || (xdt == EP_F32 && !f32))
         Py_RETURN_NONE;
     Weight w;
     if (!weight(packed, scale, cb, n, k, levels, group, w))
@@ -263,7 +258,10 @@ PyObject *backward(PyObject *, PyObject *const *args, Py_ssize_t nargs)
                 group, w))
         Py_RETURN_NONE;
     const auto opt = x2.options().requires_grad(false);
-    const auto gxt = gxdt == 0 ? at::kFloat : gxdt == 1 ? at::kHalf : gxdt == 2 ? at::kBFloat16 : x2.scalar_type();
+    const auto gxt = gxdt == EP_F32    ? at::kFloat
+                     : gxdt == EP_F16  ? at::kHalf
+                     : gxdt == EP_BF16 ? at::kBFloat16
+                                       : x2.scalar_type();
     at::Tensor out[3];
     if (need[0])
         out[0] = at::empty({m, k}, opt.dtype(gxt));
@@ -309,11 +307,11 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 {
     if (!args_are(nargs, 6))
         return nullptr;
-    fn_ws = (WorkspaceFn)PyLong_AsVoidPtr(args[0]);
-    fn_matmul = (MatmulFn)PyLong_AsVoidPtr(args[1]);
-    fn_bwd_ws = (WorkspaceFn)PyLong_AsVoidPtr(args[2]);
-    fn_backward = (BackwardFn)PyLong_AsVoidPtr(args[3]);
-    fn_error = (ErrorFn)PyLong_AsVoidPtr(args[4]);
+    fn_ws = (decltype(fn_ws))PyLong_AsVoidPtr(args[0]);
+    fn_matmul = (decltype(fn_matmul))PyLong_AsVoidPtr(args[1]);
+    fn_bwd_ws = (decltype(fn_bwd_ws))PyLong_AsVoidPtr(args[2]);
+    fn_backward = (decltype(fn_backward))PyLong_AsVoidPtr(args[3]);
+    fn_error = (decltype(fn_error))PyLong_AsVoidPtr(args[4]);
     if (PyErr_Occurred())
         return nullptr;
     fn_stream = Py_NewRef(args[5]);

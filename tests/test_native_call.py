@@ -1,9 +1,14 @@
 """The native call path from torch tensors (csrc/torch_call.cpp)."""
+import os
+import subprocess
+
 import pytest
 import torch
 
 from epure import PackedLinear, PackedWeight
 from epure.kernels import _abi, cuda
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def host_store(n=16, k=128, group=32):
@@ -51,6 +56,19 @@ def test_store_sizes_need_not_be_instance_attributes(monkeypatch):
     monkeypatch.setattr(cuda, "_AVAILABLE", True)
     s = ModuleStore(host_store())
     assert cuda.linear(torch.zeros(1, 128, dtype=torch.bfloat16), s) is None
+
+
+def test_extension_is_rebuilt_with_the_c_header():
+    """It calls the library through the header's function types: a changed
+    signature has to reach it."""
+    csrc = os.path.join(ROOT, "epure-runtime_amd", "csrc")
+    out = os.path.abspath(_abi.TORCH_PATH)
+    # -o: the other prerequisites count as old
+    r = subprocess.run(["make", "-n", "-C", csrc, "-o", "torch_call.cpp", "-o",
+                        os.path.join(ROOT, "epure-runtime_amd", "_build", "torch_id"),
+                        "-W", os.path.join(ROOT, "include", "epure_hip.h"), out],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "torch_call.cpp" in r.stdout, r.stdout + r.stderr
 
 
 # ------------------------------------------------------------------ without the extension
