@@ -223,9 +223,22 @@ void row_prep_x(const void *x, int64_t ldx, int64_t M, int64_t K, int *rexp, f16
         hipLaunchKernelGGL((row_prep_kernel<XDT, 8>), grid, block, 0, stream, x, ldx, (int)K, rexp, xh);
 }
 
-template <int BITS, int BM, int PD, int NT, int WAVES, bool GR, bool SF32, bool G128>
-__global__ void __launch_bounds__(WAVES * 64, 8 / WAVES) pf_kernel(PfArgs a)
+// Waves per SIMD that the registers have to leave room for: two workgroups
+// per CU (what the table's LDS allows) at 64 rows of eight waves and at four
+// waves, one at 128 rows.
+constexpr int pf_min_waves(int BM, int WAVES) { return BM == 64 && WAVES == 8 ? 4 : 8 / WAVES; }
+
+template <int BITS, int BM, int PF, int NT, int WAVES, bool GR, bool SF32, bool G128>
+__global__ void __launch_bounds__(WAVES * 64, pf_min_waves(BM, WAVES)) pf_kernel(PfArgs a)
 {
+    // steps of weights in flight: PF, but two where a scale load per piece
+    // and step would not leave room for the second workgroup (8-bit 64-row
+    // tiles of eight waves, groups below 128: 130 to 136 registers, one
+    // workgroup per CU).  8-bit group 64, four steps and one workgroup / two
+    // and two: 14336 x 4096 at M = 100 63.4 -> 57.4 us, 8192^2 at 127 69.8 ->
+    // 62.4, 64 x 2048 x 1024 grouped, 4096 rows 97.5 -> 79.7; four steps at
+    // two workgroups spill and took 58.5, 64.5 and 109
+    constexpr int PD = BITS == 8 && BM == 64 && WAVES == 8 && !G128 ? 2 : PF;
     constexpr int SB = SF32 ? 4 : 2;             // bytes of a group scale
     constexpr int MT = BM / 32;                  // 32-row M tiles per wave
     constexpr int THREADS = WAVES * 64;
