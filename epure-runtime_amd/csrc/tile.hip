@@ -90,71 +90,97 @@ __global__ void __launch_bounds__(256) dequant_tile_kernel(TileArgs a)
 }
 
 // The same tile for 4-bit rows of whole 16-byte chunks (K % 32 == 0, groups
-// of a multiple of 32), bound by its stores: a wave takes one row, a lane 4
-// packed bytes (8 weights, one group scale) of each 512, four loads in
-// flight, so a store instruction writes 1 KiB (2-byte types) in one piece.
-// With a thread per 32 weights its four stores lay 64 bytes from its
-// neighbours': 6144 x 2048 to fp16 beside the backward's other product 23.8
-// us, 11 to 17 now.  The codebook is pre-rounded in LDS.  Same arithmetic as
+// of a multiple of 32), bound by its stores: a wave takes 4 x 64 consecutive
+// dwords of the packed stream, a lane one dword (8 weights, one group scale)
+// of each 64, four loads in flight, so a store instruction writes 1 KiB
+// (2-byte types) in one piece wherever the rows are long enough.  With a
+// thread per 32 weights its four stores lay 64 bytes from its neighbours':
+// 6144 x 2048 to fp16 beside the backward's other product 23.8 us, 11 to 17
+// now.  The waves go over the stream and not over the rows: with a wave per
+// row a few long rows ran on a few waves (4 x 2^20 to bf16 1090 -> 6.7 us) and
+// rows shorter than 512 weights left lanes idle (2^20 x 32 365 -> 19.8 us);
+// between them 4096^2 13.8 -> 12.9, 14336 x 4096 29.6 -> 31.3.  The codebook is pre-rounded in LDS.  Same arithmetic as
 // dequant_elem (round(c) * round(s) in fp32, rounded once).
-constexpr int kTile4 = 4;  // loads in flight per lane
-template <int DT>
-__global__ void __launch_bounds__(256) dequant_tile4_kernel(TileArgs a)
+// U: dwords per lane, all loaded before the first is expanded.
+constexpr int kTile4 = 4;
+template <int DT, int U>
+__global__ void __launch_bounds__(256) dequant_tile4_kernel(TileArgs a, uint32_t dw, int64_t total)
 {
     __shared__ float tab[16];
     const int lane = threadIdx.x & 63;
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t row = n < a.N ? n : a.N - 1;  // every wave reaches the barrier
-    const int dw = (int)(a.K / 8);
-    const uint32_t *src = (const uint32_t *)(a.packed + row * (a.K / 2));
-    char *dst = (char *)a.out + row * a.ldo * (DT == EP_F32 ? 4 : 2);
-    uint32_t w[kTile4];
-    float sc[kTile4];
-    auto load = [&](int i0) {
+    const int64_t f0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * U) + lane;
+    // row and dword of the row of the lane's first dword; 64 dwords on are
+    // d64 rows and r64 dwords on
+    uint32_t row, i;
+    if (total <= 0xffffffff) {  // uniform
+        row = (uint32_t)f0 / dw;
+        i = (uint32_t)f0 - row * dw;
+    } else {
+        row = (uint32_t)(f0 / dw);
+        i = (uint32_t)(f0 - (int64_t)row * dw);
+    }
+    const uint32_t d64 = 64 / dw, r64 = 64 % dw;
+    uint32_t w[U], at[U], rows[U];
+    float sc[U];
 #pragma unroll
-        for (int u = 0; u < kTile4; ++u) {
-            const int i = min(i0 + 64 * u, dw - 1);
-            w[u] = src[i];
-            sc[u] = load_as_f32(a.scale, a.scale_dtype, row * a.lds + (uint32_t)i * 8u / (uint32_t)a.group);
+    for (int u = 0; u < U; ++u) {
+        const bool in = f0 + 64 * u < total;  // past the end: dword 0, not stored
+        rows[u] = in ? row : 0;
+        at[u] = in ? i : 0;
+        w[u] = ((const uint32_t *)a.packed)[in ? f0 + 64 * u : 0];
+        sc[u] = load_as_f32(a.scale, a.scale_dtype, (int64_t)rows[u] * a.lds + at[u] * 8u / (uint32_t)a.group);
+        row += d64;
+        i += r64;
+        if (i >= dw) {
+            i -= dw;
+            ++row;
         }
-    };
-    load(lane);
+    }
     if (threadIdx.x < 16)
         tab[threadIdx.x] = threadIdx.x < a.levels ? round_to(DT, load_as_f32(a.cb, a.cb_dtype, threadIdx.x)) : 0.0f;
     lds_barrier();
-    if (n >= a.N)
-        return;
-    for (int i0 = lane; i0 < dw; i0 += 64 * kTile4) {
 #pragma unroll
-        for (int u = 0; u < kTile4; ++u) {
-            const int i = i0 + 64 * u;
-            if (i >= dw)
-                break;
-            const float s = round_to(DT, sc[u]);
-            float v[8];
+    for (int u = 0; u < U; ++u) {
+        if (f0 + 64 * u >= total)
+            break;
+        char *dst = (char *)a.out + ((int64_t)rows[u] * a.ldo + (int64_t)at[u] * 8) * (DT == EP_F32 ? 4 : 2);
+        const float s = round_to(DT, sc[u]);
+        float v[8];
 #pragma unroll
-            for (int t = 0; t < 8; ++t)
-                v[t] = tab[(w[u] >> (4 * t)) & 15] * s;
-            if constexpr (DT == EP_F32) {
-                f32x4_t *d = (f32x4_t *)dst + (int64_t)i * 2;
-                d[0] = (f32x4_t){v[0], v[1], v[2], v[3]};
-                d[1] = (f32x4_t){v[4], v[5], v[6], v[7]};
-            } else {
-                u32x4_t o;
+        for (int t = 0; t < 8; ++t)
+            v[t] = tab[(w[u] >> (4 * t)) & 15] * s;
+        if constexpr (DT == EP_F32) {
+            ((f32x4_t *)dst)[0] = (f32x4_t){v[0], v[1], v[2], v[3]};
+            ((f32x4_t *)dst)[1] = (f32x4_t){v[4], v[5], v[6], v[7]};
+        } else {
+            u32x4_t o;
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float lo = v[2 * t], hi = v[2 * t + 1];
-                    if constexpr (DT == EP_F16)
-                        o[t] = (uint32_t)f16_bits((f16_t)lo) | ((uint32_t)f16_bits((f16_t)hi) << 16);
-                    else
-                        o[t] = (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
-                }
-                ((u32x4_t *)dst)[i] = o;
+            for (int t = 0; t < 4; ++t) {
+                const float lo = v[2 * t], hi = v[2 * t + 1];
+                if constexpr (DT == EP_F16)
+                    o[t] = (uint32_t)f16_bits((f16_t)lo) | ((uint32_t)f16_bits((f16_t)hi) << 16);
+                else
+                    o[t] = (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
             }
+            *(u32x4_t *)dst = o;
         }
-        if (i0 + 64 * kTile4 < dw)
-            load(i0 + 64 * kTile4);
     }
+}
+
+template <int DT>
+void launch_tile4(const TileArgs &a, hipStream_t stream)
+{
+    const uint32_t dw = (uint32_t)(a.K / 8);  // dwords per row
+    const int64_t total = a.N * dw;
+    // one dword per lane while four would leave fewer than two workgroups per
+    // CU: 256 x 256 to bf16 5.2 -> 4.3 us
+    if (total < (int64_t)2 * 256 * kTile4 * device_cus())
+        hipLaunchKernelGGL((dequant_tile4_kernel<DT, 1>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
+                           a, dw, total);
+    else
+        hipLaunchKernelGGL((dequant_tile4_kernel<DT, kTile4>),
+                           dim3((unsigned)((total + 256 * kTile4 - 1) / (256 * kTile4))), dim3(256), 0, stream, a, dw,
+                           total);
 }
 
 // out[i, :] = dequantized row ids[i] (epure/runtime.py:139-156
@@ -197,15 +223,14 @@ int launch_dequant_tile(const PackedDesc &w, void *out, int out_dtype, int64_t l
     const bool fast = w.levels <= 16 && w.K % 32 == 0 && w.group % 32 == 0 &&
                       ((uintptr_t)w.packed & 15) == 0 && ((uintptr_t)out & 15) == 0 &&
                       (ldo * esz) % 16 == 0 && w.K <= 0x7fffffff &&
-                      w.N <= 0x7fffffff;
+                      w.N <= 0x7fffffff && w.N * (w.K / 8) <= (int64_t)256 * kTile4 * 0x7fffffff;
     if (fast) {
-        const dim3 grid((unsigned)((w.N + 3) / 4));
         if (out_dtype == EP_F16)
-            hipLaunchKernelGGL(dequant_tile4_kernel<EP_F16>, grid, dim3(256), 0, stream, a);
+            launch_tile4<EP_F16>(a, stream);
         else if (out_dtype == EP_BF16)
-            hipLaunchKernelGGL(dequant_tile4_kernel<EP_BF16>, grid, dim3(256), 0, stream, a);
+            launch_tile4<EP_BF16>(a, stream);
         else
-            hipLaunchKernelGGL(dequant_tile4_kernel<EP_F32>, grid, dim3(256), 0, stream, a);
+            launch_tile4<EP_F32>(a, stream);
         EP_HIP_CHECK(hipGetLastError());
         return EP_OK;
     }

@@ -109,10 +109,12 @@ def test_dequant_tile_bitexact(dtype, name, levels, n, k, group):
 @pytest.mark.parametrize("dtype,name", [(torch.float32, "f32"), (torch.float16, "f16"),
                                         (torch.bfloat16, "bf16")])
 @pytest.mark.parametrize("n,k,group", [(1, 32, 32), (3, 480, 32), (4, 512, 64), (5, 544, 32),
-                                       (6, 2048, 128), (9, 2080, 32), (2, 14336, 96)])
+                                       (6, 2048, 128), (9, 2080, 32), (2, 14336, 96),
+                                       (40000, 32, 32), (33000, 160, 32), (2100, 2080, 96), (3, 1500000, 32)])
 def test_dequant_rows_bitexact(dtype, name, n, k, group):
-    """4-bit rows of whole 16-byte chunks at lengths around a wave's 512
-    weights and its 2048 in flight, and rows around four per workgroup."""
+    """4-bit rows of whole 16-byte chunks: shorter than, around and longer
+    than a wave's 512 weights, few enough weights for one dword per lane and
+    enough for four, ending inside a workgroup."""
     _, packed, scale, cb = ref.synth_linear(n, k, 16, group, seed=n + k)
     s = PackedWeight((n, k), packed, scale, cb.astype(np.float32), group, 16).to(DEV)
     w = s.materialize(dtype).float().cpu().numpy()
@@ -131,6 +133,29 @@ def test_rows_shorter_than_a_k_step(levels, n, k, group, m):
     with torch.no_grad():
         y = PackedLinear(s)(x)
     assert_close(y.float().cpu().numpy(), want, TOL + 2.0 ** -8)
+
+
+def test_dequant_time_does_not_depend_on_the_row_length():
+    """2^25 4-bit weights as a few long rows, square and as many short rows:
+    the same bytes, within four times the same time (a wave per row took
+    66 and 13 times as long at the ends)."""
+    times = []
+    for n, k in ((8192, 4096), (16, 1 << 21), (1 << 20, 32)):
+        g = torch.Generator(device=DEV).manual_seed(k)
+        s = PackedWeight((n, k), torch.randint(0, 256, (n * k // 2,), generator=g, device=DEV, dtype=torch.uint8),
+                         torch.rand(n, k // 32, generator=g, device=DEV).half(),
+                         torch.randn(16, generator=g, device=DEV), 32, 16).to(DEV)
+        best = float("inf")
+        for _ in range(6):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(10):
+                s.materialize(torch.float16)
+            e1.record()
+            e1.synchronize()
+            best = min(best, e0.elapsed_time(e1))
+        times.append(best)
+    assert max(times) < 4 * times[0], times
 
 
 # ------------------------------------------------------------------ batch-1 GEMV
