@@ -14,7 +14,7 @@
 //    straight into the B operand -- the dense weight never reaches LDS or
 //    global memory.  From M = 128 (8-bit) or 160 (4-bit): 8 waves x BM = 128
 //    (8-bit: one N tile per wave, as two would not fit 256 VGPRs; 4-bit: one
-//    tile at M < 1024, two from 1024), one workgroup per CU.  What bounds these tilings is the
+//    tile at M < 1024 and on small grids, else two), one workgroup per CU.  What bounds these tilings is the
 //    bytes a CU pulls from L2 per k step (weights + the activation tile: a
 //    CU keeps ~32 KiB of loads in flight), so wider workgroups -- more weight
 //    rows per staged activation tile -- measured faster than 4-wave ones
@@ -601,14 +601,21 @@ struct PfPlan {
 PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
 {
     PfPlan p;
-    // measured: 128 x 2 tiles lead from M = 1024 (4-bit), 128 x 1 below.  The
+    // measured: 128 x 2 tiles lead from M = 1024 (4-bit), 128 x 1 below, and
+    // above while its grid is at most one round of workgroups on rows of up
+    // to 96 steps: two tiles leave CUs idle there (f32 scales, 8192 x 1024
+    // at M = 1024 63.7 -> 40.4 us, 50.6 on the generic tiles; 2048 x 1024 at
+    // 2048 49.4 -> 34.6, 39.5; fp16 scales, 4096^2 at 1024 75.3 -> 60.9,
+    // 6144^2 115.7 -> 107.0; longer rows gain more from the wider tile:
+    // 5120 x 14336 at 1024 194 against 208).  The
     // 64-row tile on eight waves of one weight tile, two workgroups per CU
     // (four waves of two left a SIMD two waves to hide a step's lookups and
     // loads behind): 4-bit 4096^2 at M = 100 28.2 -> 24.3 us a call, 8192 x
     // 4096 at 65 31.6 -> 28.9, 8-bit 4096 x 14336 at 100 46.0 -> 40.3, 14336 x
     // 4096 at 127 48.1 -> 44.6.
     p.bm = M >= (bits == 4 ? EP_PF_BIG4_M : EP_PF_BIG8_M) ? 128 : M > 32 ? 64 : 32;
-    p.nt = p.bm == 32 || (p.bm == 128 && bits == 4 && M >= 1024) ? 2 : 1;
+    const bool one_round = ((N + 255) / 256) * ((M + 127) / 128) <= device_cus() && K <= 96 * kPfBK;
+    p.nt = p.bm == 32 || (p.bm == 128 && bits == 4 && M >= 1024 && !one_round) ? 2 : 1;
     p.waves = p.bm == 32 ? 4 : 8;
     const int bn = p.waves * 32 * p.nt;
     const int64_t tiles = ((N + bn - 1) / bn) * ((M + p.bm - 1) / p.bm);

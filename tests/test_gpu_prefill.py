@@ -212,6 +212,58 @@ def test_f32_scales_on_the_tiles(levels, group, m, n, k):
     assert_close(run(s, x).cpu().numpy(), want, 1e-4)
 
 
+def graph_us(s, x, calls=20):
+    """us a call of the packed linear's kernels, replayed as a graph."""
+    h = cuda._hot(s)
+    out = torch.empty((x.shape[0], s.out_features), device=DEV, dtype=x.dtype)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert cuda.forward(x, h, out=out) is not None
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(calls):
+            cuda.forward(x, h, out=out)
+    best = float("inf")
+    for _ in range(6):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        graph.replay()
+        e0.record()
+        graph.replay()
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 1e3 / calls)
+    return best
+
+
+@pytest.mark.parametrize("levels,m,n,k", [(16, 1024, 8192, 1024), (16, 2048, 2048, 1024)])
+def test_f32_scales_no_slower_than_the_generic_tiles(levels, m, n, k):
+    """Against the same layer with bf16 scales, which the generic MFMA kernel
+    serves: within 15% where its plan, row count or row length made the tile
+    kernel 1.2 to 2 times slower."""
+    _, _, _, _, s = make(n, k, levels, 64, seed=m + n)
+    _, x = x_bf16(m, k, m)
+    stores = [PackedWeight((n, k), s.packed, s.scale.to(dt), s.cb, 64, levels)
+              for dt in (torch.float32, torch.bfloat16)]
+    f32, generic = (graph_us(t, x) for t in stores)
+    assert f32 < 1.15 * generic, (f32, generic)
+
+
+@pytest.mark.parametrize("m,n,k", [(1024, 8192, 128), (1024, 8193, 128), (1040, 7168, 192), (2048, 4096, 6144),
+                                   (2048, 4096, 6208), (4096, 300, 512)])
+def test_one_and_two_weight_tiles(m, n, k):
+    """4-bit prompts of 1024 rows and more on both sides of the one-tile
+    rule (one round of workgroups, rows of up to 6144 values), against the
+    f64 product of the operands (fp16 x, fp16 weights).  What is left is the
+    f32 sum of K products in some order: at most K * 2^-24 = 3.7e-4 of the
+    sum of their magnitudes and far less of the result, held to 1e-4 of it."""
+    _, _, _, _, s = make(n, k, 16, 64, seed=m + n + k)
+    x = torch.randn(m, k, generator=torch.Generator(device=DEV).manual_seed(m), device=DEV).to(torch.float16)
+    want = x.double() @ s.materialize(torch.float16).double().t()
+    assert (run(s, x).double() - want).abs().max() <= 1e-4 * want.abs().max()
+
+
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("k", [64, 512, 576, 1024, 1088, 2112, 4160, 8256, 16384, 16448])
 def test_row_prep_row_lengths(k, xdt):
