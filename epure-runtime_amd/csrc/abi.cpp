@@ -68,7 +68,8 @@ static int check_weight(const PackedDesc &w)
 // ones: 4-bit 2048 x 6144 at M = 5 / 32 / 48: 92.6 / 97.1 / 113.2 -> 24.0 /
 // 27.4 / 31.5 us, 6144 x 2048 at M = 16: 36.9 -> 18.3 us, 8-bit 4096^2 at
 // M = 8: 87.4 -> 24.1 us (the tiles split K over idle CUs and look up
-// conflict-free copies of the table).
+// conflict-free copies of the table), on rows long enough for them
+// (prefill_leads_f32).
 constexpr int64_t kTileRowsMin = 4;
 
 // The workspace without which a call cannot run: any M may land on the MFMA
@@ -156,9 +157,11 @@ int ep_dequant_matmul(const void *x, int x_dtype, int64_t ldx, const uint8_t *pa
         return launch_gemv(w, xa, M, ya, s);
     if (skinny_serves(w, xa, M))
         return launch_skinny(w, xa, M, ya, workspace, workspace_bytes, s);
-    if (M > 64 && prefill_serves(w, xa, M))
+    const bool tiles = prefill_serves(w, xa, M) &&
+                       (w.scale_dtype != EP_F32 || prefill_leads_f32(w.bits(), M, N, K));
+    if (M > 64 && tiles)
         return launch_prefill(w, xa, M, ya, workspace, workspace_bytes, s);
-    if (M > kTileRowsMin && M <= 64 && w.scale_dtype == EP_F32 && prefill_serves(w, xa, M) &&
+    if (M > kTileRowsMin && M <= 64 && w.scale_dtype == EP_F32 && tiles &&
         workspace_bytes >= prefill_workspace(M, N, K, levels))
         return launch_prefill(w, xa, M, ya, workspace, workspace_bytes, s);
     if (mfma_serves(w, xa, M))

@@ -168,6 +168,10 @@ int launch_prefill(const PackedDesc &w, const ActDesc &x, int64_t M, const OutDe
 int launch_row_prep(const ActDesc &x, int64_t M, int64_t K, int *rexp, void *xh, hipStream_t stream);
 bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M);
 size_t prefill_workspace(int64_t M, int64_t N, int64_t K, int levels);
+// f32 group scales: whether the tiles lead the generic ones at this shape
+// (grouped: tile height and row length).
+bool prefill_leads_f32(int bits, int64_t M, int64_t N, int64_t K);
+bool prefill_grouped_leads_f32(int bits, int bm, int64_t K);
 
 int launch_backward(const PackedDesc &w, const ActDesc &gy, const ActDesc &x, int64_t M,
                     const OutDesc &gx, float *grad_cb, float *grad_scale, int64_t ld_gscale,

@@ -598,6 +598,12 @@ struct PfPlan {
     int bm, nt, waves, S, ksteps;
 };
 
+// Activation rows of a tile.
+int pf_rows(int bits, int64_t M)
+{
+    return M >= (bits == 4 ? EP_PF_BIG4_M : EP_PF_BIG8_M) ? 128 : M > 32 ? 64 : 32;
+}
+
 PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
 {
     PfPlan p;
@@ -613,7 +619,7 @@ PfPlan pf_plan(int bits, int64_t M, int64_t N, int64_t K)
     // loads behind): 4-bit 4096^2 at M = 100 28.2 -> 24.3 us a call, 8192 x
     // 4096 at 65 31.6 -> 28.9, 8-bit 4096 x 14336 at 100 46.0 -> 40.3, 14336 x
     // 4096 at 127 48.1 -> 44.6.
-    p.bm = M >= (bits == 4 ? EP_PF_BIG4_M : EP_PF_BIG8_M) ? 128 : M > 32 ? 64 : 32;
+    p.bm = pf_rows(bits, M);
     const bool one_round = ((N + 255) / 256) * ((M + 127) / 128) <= device_cus() && K <= 96 * kPfBK;
     p.nt = p.bm == 32 || (p.bm == 128 && bits == 4 && M >= 1024 && !one_round) ? 2 : 1;
     p.waves = p.bm == 32 ? 4 : 8;
@@ -790,6 +796,36 @@ bool prefill_serves(const PackedDesc &w, const ActDesc &x, int64_t M)
     if (((uintptr_t)w.packed & 15) != 0 || ((uintptr_t)x.ptr & 15) != 0)
         return false;
     return (x.ld * esz) % 16 == 0;
+}
+
+// f32 group scales: whether the tiles lead the generic ones, which have no
+// rescaled copy of x and no 64 KiB table to write before the first step and
+// so win short rows, less so where the weight rows alone give every CU a
+// workgroup.  Tiles / generic at N of 64 to 16384 (65536): 32-row tiles
+// 4-bit M = 32 K = 384 1.16-1.21 (0.97), 512 1.1-1.15 (0.92), 768 1.0-1.06,
+// 832 0.97-1.0; 8-bit K = 640 (1.01), 768 (0.98), 960 0.98-1.06, 1024
+// 0.66-0.78; 64-row tiles at M = 48 K = 128 0.9-1.07, 256 0.81-0.97, from M =
+// 65 0.7-0.85 at every K (there the generic kernel takes 128-row tiles);
+// 128-row tiles K = 256 (0.87-1.09), 384 0.9-1.09 (0.82-1.01), 512 4-bit
+// 0.89-1.04, 8-bit 0.9-1.08, 640 8-bit 0.83-1.03.
+bool prefill_leads_f32(int bits, int64_t M, int64_t N, int64_t K)
+{
+    const int bm = pf_rows(bits, M);
+    const int64_t steps = K / kPfBK;
+    const bool wide = (N + 255) / 256 >= device_cus();
+    if (bm == 32)
+        return steps >= (bits == 4 ? (wide ? 8 : 13) : (wide ? 12 : 16));
+    if (bm == 64)
+        return M > 64 || steps >= 4;
+    return steps >= (wide ? 6 : bits == 4 ? 8 : 10);
+}
+
+// The same for grouped experts of bm rows per tile: 32 rows 4-bit K = 128
+// 0.97-1.27, 256 0.9-1.05; 8-bit K = 256 0.9-1.14, 384 0.85-1.0; 64 rows K =
+// 128 0.78-1.15, 256 0.74-1.12; 128 rows K = 256 1.01-1.08, 384 0.95-1.04.
+bool prefill_grouped_leads_f32(int bits, int bm, int64_t K)
+{
+    return K / kPfBK >= (bm == 64 || (bm == 32 && bits == 4) ? 4 : 6);
 }
 
 // Workspace: row exponents, the fp16 activations, then the split partials;

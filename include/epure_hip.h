@@ -100,8 +100,9 @@ size_t ep_dequant_matmul_workspace(int64_t M, int64_t N, int64_t K, int levels, 
  * held in registers;
  * split-K over slices of at most 1024 otherwise; the splits' f32 partials
  * summed in split order), MFMA tiles with the weights dequantized in
- * registers above (with f32 group scales from M = 5).  Each reads the
- * packed bytes exactly once per launch.
+ * registers above (with f32 group scales from M = 5, on rows long enough
+ * for them: 256 to 1024 values by M, bits and N; the generic MFMA tiles
+ * below).  Each reads the packed bytes exactly once per launch.
  */
 int ep_dequant_matmul(const void *x, int x_dtype, int64_t ldx,
                       const uint8_t *packed, const void *scale, int scale_dtype,
@@ -135,8 +136,9 @@ int ep_expert_matmul(const void *x, int x_dtype, int64_t ldx, const int32_t *exp
  * launch whose workgroups take row tiles of one expert's tokens, each
  * reading that expert's weight rows once per tile and storing at the
  * tokens' own rows of y: the prefill MFMA kernel (32-, 64- or 128-row
- * tiles) where its shape rules hold (fp16 scales), else the generic MFMA
- * kernel (32- or 64-row tiles).
+ * tiles) where its shape rules hold (fp16 scales, or f32 ones on rows of at
+ * least 256 or 384 values), else the generic MFMA kernel (32-, 64- or
+ * 128-row tiles).
  * Replaces the reference's per-call slab materialization
  * (epure/runtime.py:163-186) and the caller's host-side grouping of tokens
  * per expert: no host synchronization, capturable in a HIP graph,

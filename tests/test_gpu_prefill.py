@@ -195,10 +195,13 @@ def test_batch1_8bit_long_k_stays_on_the_gemv():
 
 @pytest.mark.parametrize("levels,group", [(16, 128), (16, 32), (256, 128), (256, 16)])
 @pytest.mark.parametrize("m,n,k", [(5, 515, 1024), (32, 300, 512), (33, 257, 4096), (64, 256, 64),
-                                   (65, 130, 2048), (161, 513, 1088), (1024, 300, 512)])
+                                   (65, 130, 2048), (161, 513, 1088), (1024, 300, 512),
+                                   (32, 70, 832), (32, 70, 1024), (64, 70, 192), (64, 70, 256), (200, 70, 448),
+                                   (200, 70, 640)])
 def test_f32_scales_on_the_tiles(levels, group, m, n, k):
     """f32 group scales (a fine-tuned store's) on the tile kernel at the edges
-    of its row tiles (32, 64, 128), with K split and whole, against the f64
+    of its row tiles (32, 64, 128), with K split and whole, and on the generic
+    one on either side of the shortest rows the tiles take, against the f64
     product of its operands: fp16(fp16(cb) * fp16(scale)) and x, exact in
     fp16.  What is left is the f32 sum of K <= 4096 products in some order,
     at most K * 2^-24 = 2.5e-4 of the sum of their magnitudes and far less of
@@ -237,7 +240,8 @@ def graph_us(s, x, calls=20):
     return best
 
 
-@pytest.mark.parametrize("levels,m,n,k", [(16, 1024, 8192, 1024), (16, 2048, 2048, 1024)])
+@pytest.mark.parametrize("levels,m,n,k", [(16, 1024, 8192, 1024), (16, 2048, 2048, 1024), (16, 32, 2048, 64),
+                                          (256, 32, 512, 512), (256, 5, 8192, 256), (256, 2048, 512, 128)])
 def test_f32_scales_no_slower_than_the_generic_tiles(levels, m, n, k):
     """Against the same layer with bf16 scales, which the generic MFMA kernel
     serves: within 15% where its plan, row count or row length made the tile
