@@ -135,6 +135,19 @@ def test_backward_library_route_vs_closed_forms(n, k, m, group):
     assert all(torch.equal(p, q) for p, q in zip((gx, gcb, gsc), again))   # deterministic
 
 
+def test_backward_past_the_library_route():
+    """A product of more than 2^35 multiply-adds: the fused kernels at more
+    than 512 tokens."""
+    n, k, m = 4096, 4224, 2064
+    _, _, _, _, s = make(n, k, seed=41)
+    x, gy = bf16((m, k), 42), bf16((m, n), 43, 1e-2)
+    gx, gcb, gsc = run_bwd(s, gy, x)
+    wgx, wgcb, wgsc = closed_forms_t64(gy, x, s)
+    assert rel(gx.float(), wgx) < 2e-3
+    assert rel(gsc, wgsc) < 1e-4
+    assert rel(gcb, wgcb) < 1e-4
+
+
 @pytest.mark.parametrize("n,k", [(2048, 6144), (6144, 2048)])
 def test_backward_config4(n, k):
     _, packed, _, _, s = make(n, k, seed=7)
