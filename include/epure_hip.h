@@ -235,10 +235,13 @@ int ep_read_probe(const void *buf, int64_t bytes, uint32_t *sink, int grid, void
  * kernels allocate their outputs per call.  Same arguments, semantics and
  * return codes as ep_dequant_matmul; the workspace is a static device array
  * of ep_noalloc_scratch_bytes() bytes (32 MiB) per GPU, kept until the
- * process ends.  Shapes whose ep_dequant_matmul_workspace exceeds it are
- * rejected with EP_ERR_WORKSPACE before any launch.  Nothing is allocated
- * and nothing in the scratch must start at zero; calls that overlap on one
- * GPU (two streams or threads at once) race on the shared scratch.
+ * process ends.  Shapes that cannot run in it are rejected with
+ * EP_ERR_WORKSPACE before any launch: what ep_dequant_matmul_workspace asks
+ * for, but at M = 5..64 without what the tiles would add for f32 group scales
+ * (those then run on the generic kernel, the same f32 sums in another order).
+ * Nothing is allocated and nothing in the scratch must start at zero; calls
+ * that overlap on one GPU (two streams or threads at once) race on the shared
+ * scratch.
  */
 size_t ep_noalloc_scratch_bytes(void);
 int ep_dequant_matmul_noalloc(const void *x, int x_dtype, int64_t ldx,

@@ -19,7 +19,7 @@ def experts(E, n, k, levels, group, seed):
     idx = rng.integers(0, levels, E * n * k).astype(np.uint8)
     packed = ref.pack4(idx, levels)
     cb = np.sort(rng.standard_normal(levels)).astype(np.float16).astype(np.float32)
-    scale = (np.abs(rng.normal(0, 0.02, (E * n, k // group))) + 1e-3).astype(np.float16)
+    scale = (np.abs(rng.normal(0, 0.02, (E * n, -(-k // group)))) + 1e-3).astype(np.float16)
     s = PackedWeight((E, n, k), packed, scale, cb, group, levels).to(DEV)
     return s, packed, scale, cb
 
@@ -297,10 +297,10 @@ def test_grouped_experts_graph_replay_follows_ids(E, T, k):
 
 
 @pytest.mark.parametrize("E,T", [(6, 40), (3, 200)])
-def test_grouped_experts_f32_scales_generic_kernel(E, T):
-    """float32 group scales and a bfloat16 codebook (after make_trainable)
-    take the generic MFMA kernel over the sorted runs (32- / 64-row tiles;
-    per-expert scale stride in 4-byte units)."""
+def test_grouped_experts_f32_scales_bf16_codebook(E, T):
+    """float32 group scales (after make_trainable) and a bfloat16 codebook
+    on the prefill tiles (32 and 64 rows): the per-expert scale stride in
+    4-byte units."""
     n, k, group = 256, 1024, 128
     rng = np.random.Generator(np.random.PCG64(31 + T))
     idx = rng.integers(0, 16, E * n * k).astype(np.uint8)
@@ -342,13 +342,49 @@ def test_grouped_experts_clamp_ids_and_strided_rows():
 @pytest.mark.parametrize("E,n,k,T", [(3, 130, 128, 100), (3, 515, 1088, 330), (40, 1700, 192, 1300),
                                      (40, 1665, 128, 4000), (3, 131, 320, 61), (40, 1700, 192, 900)])
 def test_grouped_row_tiles(levels, E, n, k, T):
+    grouped_case(levels, E, n, k, T, 64)
+
+
+@pytest.mark.parametrize("levels", [16, 256])
+@pytest.mark.parametrize("E,n,k,T", [(3, 130, 192, 100), (3, 515, 1088, 330), (40, 1700, 192, 1300),
+                                     (40, 1665, 320, 4000), (3, 131, 320, 61), (40, 1700, 192, 900)])
+def test_grouped_row_tiles_of_scale_pairs(levels, E, n, k, T):
+    """The same with groups of 128, whose one scale load serves two steps, an
+    odd number of steps leaving the last pair half used; the wide eight-wave
+    tile and the wide 32-row one among them."""
+    grouped_case(levels, E, n, k, T, 128)
+
+
+@pytest.mark.parametrize("levels,group", [(16, 64), (16, 128), (256, 16), (256, 64), (256, 128)])
+@pytest.mark.parametrize("E,n,k,T", [(3, 130, 448, 61), (3, 130, 448, 200), (40, 1700, 384, 900),
+                                     (40, 1700, 448, 1300), (3, 130, 384, 500)])
+def test_grouped_row_tiles_f32_scales(levels, group, E, n, k, T):
+    """f32 group scales at every tile height (32, 64, 128 rows), narrow and
+    wide: fp16 scale values stored as f32, so the weights are the same."""
+    grouped_case(levels, E, n, k, T, group, np.float32)
+
+
+@pytest.mark.parametrize("levels", [16, 256])
+@pytest.mark.parametrize("scale_dt,group,k", [(np.float16, 96, 576), (np.float32, 96, 576), (np.float32, 64, 192)])
+@pytest.mark.parametrize("E,n,T", [(6, 130, 100), (3, 130, 150), (3, 257, 500)])
+def test_grouped_generic_kernel(levels, scale_dt, group, k, E, n, T):
+    """What the prefill tiles do not take, at every tile height of the
+    generic grouped kernel (32, 64, 128 rows): groups that are no power of
+    two, and f32 scales on short rows."""
+    grouped_case(levels, E, n, k, T, group, scale_dt)
+
+
+def grouped_case(levels, E, n, k, T, group, scale_dt=np.float16):
     """Experts of 32 to 127 mean rows (64-row tiles) and fewer (32-row tiles)
     on both sides of the workgroup width's rule (few weight rows in all: 128 per workgroup, else
     256), rows of a run ending inside a tile and N inside a workgroup, against
     the f64 product of the operands: fp16 x as it is and fp16 weights, so what
     is left is the f32 sums (K <= 1088 products, at most 1088 * 2^-24 = 6.5e-5
     of their magnitudes) and the fp16 output's 2^-11."""
-    s, packed, scale, cb = experts(E, n, k, levels, 64, seed=E + n)
+    print(f"case: grouped {E} x {n} x {k} rows={T} levels={levels} group={group} {scale_dt.__name__}", flush=True)
+    s, packed, scale, cb = experts(E, n, k, levels, group, seed=E + n)
+    if scale_dt is np.float32:
+        s.scale = s.scale.float()
     g = torch.Generator(device=DEV).manual_seed(T)
     x = torch.randn(T, k, generator=g, device=DEV).to(torch.float16)
     ids = torch.randint(0, E, (T,), generator=g, device=DEV)

@@ -165,3 +165,28 @@ def _random_x(k, xdt):
     g = torch.Generator()
     g.manual_seed(k)
     return torch.randn(1, k, generator=g).to(DEV).to(xdt)
+
+
+@pytest.mark.parametrize("levels,k,n", [(16, 2048, 28673), (16, 6144, 7177), (16, 12288, 6149), (256, 3072, 7177),
+                                        (256, 6144, 12293), (256, 14336, 6149)])
+@pytest.mark.parametrize("scale_dt", [torch.float32, torch.bfloat16])
+def test_row_gemv_streamed_blocks_of_other_scales(levels, k, n, scale_dt):
+    """The streamed form with f32 and bf16 group scales (their own
+    instantiation and conversion), rows of 12, 24 and 56 slabs, and results
+    added to a 16-bit y: against the f64 product of the operands plus y, the
+    sum rounded to y's type once."""
+    packed, scale, cb = _random_store(n, k, levels)
+    s = PackedWeight((n, k), packed, scale.to(scale_dt), cb, 128, levels).to(DEV)
+    print(f"case: streamed row GEMV N={n} K={k} levels={levels} scales={scale_dt}", flush=True)
+    x = _random_x(k, torch.float16)
+    y0 = torch.randn(1, n, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV).half()
+    y = cuda.forward(x, cuda._hot(s), out=y0.clone(), accumulate=True)
+    assert y is not None, f"declined: {_abi.last_error()}"
+    idx = s.packed.view(n, -1)
+    if levels == 16:
+        idx = torch.stack((idx & 15, idx >> 4), dim=-1).view(n, k)
+    w = s.cb.double()[idx.long()] * s.scale.double().repeat_interleave(128, dim=1)
+    want = x.double() @ w.t() + y0.double()
+    # y's own rounding, 2^-11 of it, beside the sums' 1e-4 of the rms
+    err = (y.double() - want).abs() - 2.0 ** -11 * want.abs()
+    assert err.max() <= 1e-4 * want.pow(2).mean().sqrt()

@@ -4,8 +4,10 @@ import subprocess
 
 import pytest
 import torch
+import torch.nn.utils.parametrize
+import torch.utils._python_dispatch
 
-from epure import PackedLinear, PackedWeight
+from epure import PackedLinear, PackedWeight, make_trainable
 from epure.kernels import _abi, cuda
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -108,3 +110,158 @@ def test_calls_without_the_extension_are_the_same(monkeypatch):
     for a, b in zip(results(), native):
         assert a.dtype == b.dtype and torch.equal(a, b)
     assert cuda.backward(gy.float(), x2, h) is None          # declined on both
+
+
+# ------------------------------------------------------------------ linear, on the GPU
+DEV = torch.device("cuda:0")
+
+
+def gpu_linear(levels=16, n=144, k=256, group=32):
+    g = torch.Generator().manual_seed(levels + k)
+    packed = torch.randint(0, 256, (n * k // (1 if levels > 16 else 2),), generator=g, dtype=torch.uint8)
+    scale = (torch.rand(n, k // group, generator=g) + 0.1).half()
+    return PackedLinear(PackedWeight((n, k), packed, scale, torch.randn(levels, generator=g), group, levels)).to(DEV)
+
+
+def rows(m, k, dtype, seed=3):
+    return torch.randn(m, k, generator=torch.Generator(device=DEV).manual_seed(seed), device=DEV).to(dtype)
+
+
+def direct(lin, x):
+    """What the kernels give for the contiguous rows of x."""
+    y = cuda.forward(x.reshape(-1, x.shape[-1]).contiguous(), cuda._hot(lin.store))
+    return y.view(*x.shape[:-1], -1)
+
+
+def call(x, s):
+    return _abi.call.linear(x, s.packed, s.scale, s.cb, s.out_features, s.in_features, s.levels, s.group,
+                            cuda.SERVE_F32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("levels", [16, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_takes_every_layout(levels, dtype):
+    """1-D to 4-D x, a transposed one, every second column, rows further
+    apart than K, a slice at an offset: the kernels' result for the same rows
+    (bit for bit; with rows apart the same kernels run), in x's shape."""
+    lin = gpu_linear(levels)
+    k = lin.store.in_features
+    x = rows(24, k, dtype)
+    wide = rows(24, k + 8, dtype, 4)
+    for v in (x[0], x[:1], x, x.view(2, 12, k), x.view(2, 3, 4, k), rows(k, 24, dtype, 5).t(),
+              rows(24, 2 * k, dtype, 6)[:, ::2], wide[:, :k], wide[:, 8:], x[8:20], x.view(2, 12, k)[:, :5]):
+        with torch.no_grad():
+            y = lin(v)
+        assert y.shape == (*v.shape[:-1], 144) and y.dtype == dtype and not y.requires_grad
+        assert torch.equal(y, direct(lin, v)), (v.shape, v.stride())
+
+
+@pytest.mark.gpu
+def test_linear_serves_f32_only_when_asked(monkeypatch):
+    lin = gpu_linear()
+    x = rows(5, 256, torch.float32)
+    with torch.no_grad():
+        assert cuda.linear(x, lin.store) is None
+        assert cuda.linear(x.to(torch.float64), lin.store) is None
+        monkeypatch.setattr(cuda, "SERVE_F32", True)
+        assert torch.equal(cuda.linear(x, lin.store), direct(lin, x))
+
+
+@pytest.mark.gpu
+def test_linear_runs_on_the_current_stream():
+    lin = gpu_linear()
+    x = rows(40, 256, torch.bfloat16)
+    want = direct(lin, x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(side):
+        v = torch.zeros_like(x)
+        for _ in range(50):      # the product is behind these on its stream, or reads zeros
+            v.copy_(torch.zeros_like(x))
+        v.copy_(x)
+        y = lin(v)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+
+
+@pytest.mark.gpu
+def test_linear_reports_the_library_error():
+    """Rows that overlap: refused by the library, as an exception."""
+    lin = gpu_linear()
+    x = rows(1, 256, torch.bfloat16).expand(8, 256)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="ep_dequant_matmul failed.*row length"):
+        lin(x)
+
+
+class Wrapped(torch.Tensor):
+    pass
+
+
+class FunctionMode(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class DispatchMode(torch.utils._python_dispatch.TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+def test_linear_hands_back_what_torch_wants_to_see():
+    """A tensor subclass, function and dispatch modes, a wrong or empty row
+    and autograd take the path through torch's operators."""
+    lin = gpu_linear()
+    s, x = lin.store, rows(6, 256, torch.bfloat16)
+    want = direct(lin, x)
+    with torch.no_grad():
+        assert torch.equal(call(x, s), want)
+        assert call(x.as_subclass(Wrapped), s) is NotImplemented
+        assert call(x[:, :128], s) is NotImplemented
+        assert call(x[:0], s) is NotImplemented and lin(x[:0]).shape == (0, 144)
+        for mode in (FunctionMode(), DispatchMode()):
+            with mode:
+                assert call(x, s) is NotImplemented
+                y = lin(x)
+            assert torch.equal(y, want)
+        assert torch.equal(lin(x.as_subclass(Wrapped)).as_subclass(torch.Tensor), want)
+    seen = []
+    with torch.no_grad():
+        torch.vmap(lambda v: seen.append(call(v, s)) or v)(x.view(2, 3, 256))
+    assert seen == [NotImplemented]
+    assert torch.equal(call(x, s), want)                  # grad mode, nothing requires grad
+    assert call(x.clone().requires_grad_(True), s) is NotImplemented
+
+
+@pytest.mark.gpu
+def test_linear_of_a_trainable_store():
+    """Without grad mode the native call; with it the autograd function."""
+    lin = gpu_linear()
+    make_trainable(torch.nn.Sequential(lin), "both", verbose=False)
+    x = rows(6, 256, torch.bfloat16)
+    with torch.no_grad():
+        y = lin(x)
+        assert call(x, lin.store) is not NotImplemented
+    assert call(x, lin.store) is NotImplemented
+    z = lin(x)
+    assert z.requires_grad and torch.equal(z.detach(), y)
+    z.float().sum().backward()
+    assert lin.store.scale.grad is not None and lin.store.cb.grad is not None
+
+
+class Doubled(torch.nn.Module):
+    def forward(self, t):
+        return 2 * t
+
+
+@pytest.mark.gpu
+def test_linear_of_a_parametrized_store():
+    """A store whose scale is computed: its value, not a kept tensor."""
+    lin = gpu_linear()
+    x = rows(6, 256, torch.bfloat16)
+    with torch.no_grad():
+        y = lin(x)
+        torch.nn.utils.parametrize.register_parametrization(lin.store, "scale", Doubled())
+        assert torch.equal(lin(x), 2 * y)

@@ -1,7 +1,8 @@
 """ep_dequant_matmul_noalloc (static device scratch, no allocation) against
-ep_dequant_matmul with a caller workspace: the same kernels run, so the
-outputs must be bit-identical; both are also held to the Rust-order oracle
-bar (max relative error 2e-3).  Two calls in a row, the second smaller, so a
+ep_dequant_matmul with a caller workspace: the same kernels run wherever the
+scratch holds the workspace they ask for, so the outputs must be
+bit-identical; both are also held to the Rust-order oracle bar (max relative
+error 2e-3).  Two calls in a row, the second smaller, so a
 stale scratch from the first call cannot leak into the second."""
 import numpy as np
 import pytest
@@ -76,3 +77,19 @@ def test_noalloc_rejects_requests_beyond_the_scratch():
         None, _abi.BF16, 512, None, None, _abi.F16, 4, None, _abi.F32, 16, 128, 1, 256, 512,
         None, _abi.F32, 256, 0, _abi.stream_handle(DEV))
     assert rc == -1 and "null" in _abi.last_error()
+
+
+def test_noalloc_f32_scales_past_the_tiles_workspace():
+    """f32 group scales where the tiles' split partials exceed the scratch but
+    the generic tiles' row exponents do not: served by the generic kernel, in
+    another order of the same f32 sums (K = 4096 products: at most 2.5e-4 of
+    their magnitudes, far less of the largest result, held to 1e-4 of it)."""
+    n, k, m = 16384, 4096, 64
+    assert _abi.lib.ep_dequant_matmul_workspace(m, n, k, 16, 128) > _abi.lib.ep_noalloc_scratch_bytes()
+    g = torch.Generator(device=DEV).manual_seed(3)
+    s = PackedWeight((n, k), torch.randint(0, 256, (n * k // 2,), generator=g, device=DEV, dtype=torch.uint8),
+                     torch.rand(n, k // 128, generator=g, device=DEV) + 0.01, torch.randn(16, generator=g, device=DEV),
+                     128, 16).to(DEV)
+    x = torch.randn(m, k, generator=g, device=DEV).to(torch.bfloat16)
+    a, b = _run(s, x, noalloc=True), _run(s, x, noalloc=False)
+    assert np.abs(a - b).max() <= 1e-4 * np.abs(b).max()
