@@ -333,7 +333,7 @@ def prefill_sweep(seed=0, replays=10):
                                     if _sk2_serves(m, n, k) else
                                     "sk1_kernel" if _sk1_serves(m, n, cus) else
                                     "sk_kernel + sk_reduce_kernel" if m <= 64 else
-                                    "pf_prep_kernel + pf_kernel (+ sk_reduce_kernel when K is split)")})
+                                    "row_prep_kernel + pf_kernel (+ sk_reduce_kernel when K is split)")})
             del lins, x
         del stores
         torch.cuda.empty_cache()
@@ -647,9 +647,9 @@ def side_workload(args):
         # kernels, the two chains on two streams; --fused-backward the fused kernels
         out["config"]["route"] = "fused" if args.fused_backward else "library"
         out["roofline"] = {"bound": "mfma",
-                           "kernel": ("gy_prep_kernel + dx_kernel + dw_kernel + gc_final_kernel"
+                           "kernel": ("row_prep_kernel + dx_kernel + dw_kernel + gc_final_kernel"
                                       if args.fused_backward else
-                                      "hipBLASLt GEMMs + gy_prep/dequant_tile4/dx_finish/gw_epilogue/gc_final"),
+                                      "hipBLASLt GEMMs + row_prep/dequant_tile4/dx_finish/gw_epilogue/gc_final"),
                            "achieved": round(tf, 2), "peak": MFMA_PEAK_TFLOPS,
                            "unit": "TFLOP/s", "frac": round(tf / MFMA_PEAK_TFLOPS, 4),
                            "traffic": None}
