@@ -628,8 +628,8 @@ __global__ void __launch_bounds__(512) gemv_lut_kernel(GemvArgs a)
 // during this one's products: the per-block prologue (64 KiB of table for 32
 // KiB of weights) was most of a long layer's time, and then the rows' lane
 // sums (now shared by a wave's rows: 12 instead of 48 operations for four).
-// 4-bit 151936 x 2048 50.5 -> 33.3 us (4.8 TB/s; 42.2 before the shared
-// sums), 32768 x 8192 57.2 -> 28.9, 8192^2 16.1 -> 10.5, 8-bit 28672 x 4096
+// 4-bit 151936 x 2048 50.5 -> 30.6 us (graph replays over weights no cache
+// holds, 5.2 TB/s; 42.2 before the shared sums), 32768 x 8192 57.2 -> 28.9, 8192^2 16.1 -> 10.5, 8-bit 28672 x 4096
 // 33.0 -> 24.6.
 template <int BITS, int XDT, int S, bool SC32, int MT, bool LOOP>
 __global__ void __launch_bounds__(64 * EP_GEMV_ROW_WAVES, LOOP ? 4 : 1) gemv_row_kernel(GemvArgs a)

@@ -685,7 +685,7 @@ size_t prefill_grouped_workspace(int64_t T, int64_t K)
 
 // Stacked experts grouped by expert (tiles from the device sort): the fp16
 // copy of every token row, then pf_kernel over each expert's row tiles (bm
-// 64 or 128 rows, the whole K per workgroup), results at the tokens' rows.
+// 32, 64 or 128 rows, the whole K per workgroup), results at the tokens' rows.
 int launch_prefill_grouped(const PackedDesc &w, const ActDesc &x, int64_t T, const int *perm,
                            const int *tiles, const int *ntiles, int64_t experts, int bm, unsigned tiles_y,
                            const OutDesc &y, void *ws, hipStream_t stream)

@@ -50,8 +50,8 @@ _BUFFER_CACHE = {}
 # materialize + a dense GEMM (reference runtime.py:26-31 defaults to 8 on
 # A100).  On MI355X the fused kernels win at every measured row count of
 # the 8-bit config-3 sweep (M = 1..2048 at 4096x4096, 14336x4096,
-# 4096x14336) but one near-tie (M = 2048 at 14336x4096: 386 vs 368 us), so
-# unset every row count stays on the fused kernels.
+# 4096x14336; closest at M = 2048, 14336x4096: 349 against 367 us), so unset
+# every row count stays on the fused kernels.
 _DENSE_ABOVE = int(os.environ.get("EPURE_DENSE_ABOVE", str(2**31 - 1)))
 
 _TABLE = 256  # entries of the level table (the largest codebook an index can address)

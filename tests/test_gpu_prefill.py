@@ -128,8 +128,8 @@ def test_prefill_x_dtypes(xdt):
 @pytest.mark.parametrize("m", [80, 300])
 @pytest.mark.parametrize("group,levels", [(32, 16), (64, 16), (16, 256), (256, 256), (96, 16), (48, 256)])
 def test_prefill_groups(group, levels, m):
-    """Both tilings: 64 activation rows x 64 weight rows per wave, and 128
-    activation rows x 32 weight rows per wave (M >= 256).  Groups that
+    """Both tilings: 64 and 128 activation rows (from M = 160 at 4 bits, 128
+    at 8), each x 32 weight rows per wave.  Groups that
     neither divide the 64-wide k step nor are 64 * 2^i (96, 48) are served by
     the generic MFMA path."""
     n, k = 300, 1024 if 1024 % group == 0 else 1152
