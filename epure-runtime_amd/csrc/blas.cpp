@@ -22,6 +22,7 @@
 // later shapes of the bucket take it when the heuristic offers it for
 // them, else the heuristic's first choice, with no timing and no host
 // wait.  A plan made during capture takes the heuristic's first choice.
+// Only algorithms that fit the workspace count among the heuristic's.
 // Matrices are column-major in hipBLASLt's terms; callers pass row-major
 // buffers as their transposes.
 #include <hip/hip_runtime.h>
@@ -177,6 +178,14 @@ int make_plan(Plan &p, hipblasLtHandle_t h, const float *alpha, const void *A, c
     hipblasLtMatmulPreferenceDestroy(pref);
     if (s != HIPBLAS_STATUS_SUCCESS)
         return set_error(EP_ERR_HIP, "hipblasLtMatmulAlgoGetHeuristic: %s", status_name(s));
+    // the heuristic also returns algorithms that need more than the limit it
+    // was given (40 to 56 MiB of 32 for 2048 x 14336 x 4096): they would
+    // write past the caller's workspace
+    int fit = 0;
+    for (int i = 0; i < nres; ++i)
+        if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= p.ws)
+            res[fit++] = res[i];
+    nres = fit;
     if (nres < 1)
         return set_error(EP_DECLINE_SHAPE, "hipBLASLt has no algorithm for this GEMM");
     p.algo = res[0].algo;

@@ -135,6 +135,34 @@ def test_backward_library_route_vs_closed_forms(n, k, m, group):
     assert all(torch.equal(p, q) for p, q in zip((gx, gcb, gsc), again))   # deterministic
 
 
+@pytest.mark.parametrize("m,n,k", [(512, 14336, 4096), (1024, 8192, 4096)])
+def test_backward_stays_inside_its_workspace(m, n, k):
+    """The first call of a shape bucket times the library's candidates, some
+    of which ask for up to 56 MiB whatever the limit: nothing may be written
+    past the workspace the caller passes (here the head of a longer buffer).
+    The second call runs the two chains at once."""
+    g = torch.Generator(device=DEV).manual_seed(m)
+    packed = torch.randint(0, 256, (n * k // 2,), generator=g, device=DEV, dtype=torch.uint8)
+    scale = torch.rand(n, k // 128, generator=g, device=DEV) + 0.01
+    cb = torch.randn(16, generator=g, device=DEV)
+    x, gy = bf16((m, k), 51), bf16((m, n), 52, 1e-2)
+    gx, gcb, gsc = torch.empty(m, k, device=DEV), torch.empty(16, device=DEV), torch.empty(n, k // 128, device=DEV)
+    need = _abi.lib.ep_dequant_matmul_bwd_workspace(m, n, k, 16, 128)
+    assert need > n * k * 6 + (64 << 20)                     # the library route's
+    buf = torch.full((need + (64 << 20),), 0xA5, device=DEV, dtype=torch.uint8)
+    for _ in range(2):
+        print(f"case: backward workspace M={m} N={n} K={k}", flush=True)
+        rc = _abi.lib.ep_dequant_matmul_bwd(
+            gy.data_ptr(), _abi.BF16, n, x.data_ptr(), _abi.BF16, k, packed.data_ptr(), scale.data_ptr(), _abi.F32,
+            k // 128, cb.data_ptr(), _abi.F32, 16, 128, m, n, k, gx.data_ptr(), _abi.F32, k, gcb.data_ptr(),
+            gsc.data_ptr(), k // 128, buf.data_ptr(), need, _abi.stream_handle(DEV))
+        assert rc == 0, _abi.last_error()
+        torch.cuda.synchronize()
+        assert bool((buf[need:] == 0xA5).all())
+    w = dense_tile(packed, scale, cb, n, k, 128, 16)
+    assert rel(gx, gy.double() @ w.double()) < 2e-3
+
+
 def test_backward_past_the_library_route():
     """A product of more than 2^35 multiply-adds: the fused kernels at more
     than 512 tokens."""
