@@ -694,13 +694,6 @@ static int dx_splits(int64_t M, int64_t N, int64_t K)
 // handle, no host wait, at about half the library route's rate at 2048
 // tokens.
 constexpr int64_t kBlasMinM = 512;
-// Multiply-adds of one product up to which the library route runs: the
-// largest that have run here (2048 x 4096^2, 1024 x 8192 x 4096).  The first
-// call of 2048 x 14336 x 4096, of which only the library's products and the
-// timing of their candidates are new beside those, ended in a GPU fault
-// whose cause is not known; larger products stay on the fused kernels (369
-// against 650 TFLOP/s at 2048 x 6144 x 2048) until it is.
-constexpr int64_t kBlasMaxProduct = (int64_t)1 << 35;
 static bool fused_forced()
 {
     static const bool forced = [] {
@@ -711,7 +704,7 @@ static bool fused_forced()
 }
 static bool blas_route(int64_t M, int64_t N, int64_t K)
 {
-    return M >= kBlasMinM && N >= 256 && K >= 256 && M <= kBlasMaxProduct / (N * K) && !fused_forced();
+    return M >= kBlasMinM && N >= 256 && K >= 256 && !fused_forced();
 }
 static size_t al256(size_t b) { return (b + 255) / 256 * 256; }
 

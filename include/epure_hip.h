@@ -163,11 +163,11 @@ int ep_expert_matmul_grouped(const void *x, int x_dtype, int64_t ldx, const int3
  * overwritten, not accumulated, and are deterministic (fixed-order
  * reductions).  `packed` is only read.
  * Two routes, chosen by shape:
- *   M < 512, N or K < 256, or M N K > 2^35: the fused kernels.  Each grad_W
- *     tile stays in registers and is reduced against the codebook in place:
- *     neither W nor grad_W is written to memory; the workspace holds per-row
- *     exponents, an fp16 copy of gy and grad_x split partials.
- *   else library GEMMs.  The workspace receives W materialized as fp16
+ *   M < 512 (or N, K < 256): the fused kernels.  Each grad_W tile stays in
+ *     registers and is reduced against the codebook in place: neither W nor
+ *     grad_W is written to memory; the workspace holds per-row exponents,
+ *     an fp16 copy of gy and grad_x split partials.
+ *   M >= 512: library GEMMs.  The workspace receives W materialized as fp16
  *     [N, K] and grad_W = gy^T . x as f32 [N, K] (written once, read once by
  *     the epilogue that forms grad_scale and grad_cb), plus the fp16 gy, an
  *     f32 [M, K] grad_x product and two 32 MiB hipBLASLt workspaces.

@@ -135,7 +135,7 @@ def test_backward_library_route_vs_closed_forms(n, k, m, group):
     assert all(torch.equal(p, q) for p, q in zip((gx, gcb, gsc), again))   # deterministic
 
 
-@pytest.mark.parametrize("m,n,k", [(512, 14336, 4096), (1024, 8192, 4096)])
+@pytest.mark.parametrize("m,n,k", [(512, 14336, 4096), (1024, 8192, 4096), (2048, 14336, 4096)])
 def test_backward_stays_inside_its_workspace(m, n, k):
     """The first call of a shape bucket times the library's candidates, some
     of which ask for up to 56 MiB whatever the limit: nothing may be written
@@ -161,19 +161,6 @@ def test_backward_stays_inside_its_workspace(m, n, k):
         assert bool((buf[need:] == 0xA5).all())
     w = dense_tile(packed, scale, cb, n, k, 128, 16)
     assert rel(gx, gy.double() @ w.double()) < 2e-3
-
-
-def test_backward_past_the_library_route():
-    """A product of more than 2^35 multiply-adds: the fused kernels at more
-    than 512 tokens."""
-    n, k, m = 4096, 4224, 2064
-    _, _, _, _, s = make(n, k, seed=41)
-    x, gy = bf16((m, k), 42), bf16((m, n), 43, 1e-2)
-    gx, gcb, gsc = run_bwd(s, gy, x)
-    wgx, wgcb, wgsc = closed_forms_t64(gy, x, s)
-    assert rel(gx.float(), wgx) < 2e-3
-    assert rel(gsc, wgsc) < 1e-4
-    assert rel(gcb, wgcb) < 1e-4
 
 
 @pytest.mark.parametrize("n,k", [(2048, 6144), (6144, 2048)])
